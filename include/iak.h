@@ -46,7 +46,7 @@
  *   iak_dense_attention         dense_attention() reference.py:16-45 (causal, mask, original_kv_positions),
  *                               under semantic_block_attention() reference.py:81-129 and
  *                               intent_quant_attention_reference() intent_quant_attention.py:20-119
- *   iak_dense_attention_workspace (no counterpart: sizes the optional split-over-keys partial buffer)
+ *   iak_dense_attention_workspace (no counterpart: sizes the optional split-over-keys and tile-flag buffer)
  *   iak_fake_quant_blocks       the per-block fake_quantize_tensor() reconstructions and their torch.cat
  *                               in intent_quant_attention_reference() intent_quant_attention.py:56-84
  *                               (intent_quant.py:221-312), float32 K and V
@@ -520,13 +520,14 @@ iak_status iak_mla_decode_rows(const iak_mla_rows_args* args, void* workspace, s
  *        mask_dtype IAK_DTYPE_* or IAK_MASK_BOOL (one byte)
  *   kv_positions [kv_len] int64 (IAK_CAUSAL_POSITIONS only)
  *   head_dim, v_dim <= 1024; kv_len <= INT32_MAX - 4096.
- * workspace (may be NULL): with it, a call with few rows and many keys splits
- * each row's keys over several workgroups and merges their partials in a
- * second kernel; it must then hold iak_dense_attention_workspace() bytes
- * (16-byte aligned; 0 bytes means the shape is not split and the workspace is
+ * workspace (may be NULL): with it, calls with several query rows per batch entry
+ * and 16-byte aligned rows run on the matrix cores, and a call with few rows and
+ * many keys splits each row's keys over several workgroups and merges their
+ * partials in a second kernel; it must then hold iak_dense_attention_workspace()
+ * bytes (16-byte aligned; 0 bytes means neither applies and the workspace is
  * unused). Without it every row runs in one workgroup. The results agree to
- * float32 rounding of the summation order. Calls that share a workspace on
- * different streams race. */
+ * float32 rounding of the summation order, NaN and infinities included. Calls
+ * that share a workspace on different streams race. */
 enum { IAK_MASK_BOOL = 3 };
 enum { IAK_CAUSAL_NONE = 0, IAK_CAUSAL_TRIU = 1, IAK_CAUSAL_POSITIONS = 2 };
 typedef struct {
@@ -541,7 +542,8 @@ typedef struct {
   float sm_scale;
 } iak_dense_attention_args;
 
-/* Bytes of device workspace that lets iak_dense_attention split these rows (0: no split). */
+/* Bytes of device workspace that lets iak_dense_attention split these rows or run them on
+ * the matrix cores (0: neither). */
 iak_status iak_dense_attention_workspace(const iak_dense_attention_args* args, size_t* bytes);
 
 iak_status iak_dense_attention(const iak_dense_attention_args* args, void* workspace, size_t workspace_bytes,

@@ -13,6 +13,11 @@
 // every product and sum is float32 over float32, float16 or bfloat16 inputs,
 // and the output is rounded once to the input dtype.
 //
+// Calls with several query rows per batch entry run on the matrix cores
+// (dense_matrix.h: causal prefill of 32 heads x 2,048 rows x 128 in float16
+// 10.8 ms -> 0.10 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 18 us);
+// what follows is the rows form, for the rest.
+//
 // Work split. A (batch, query) row's keys go to `splits` workgroups of
 // consecutive key ranges (`chunk` keys each); splits > 1 only when the caller
 // gives a workspace and there are few rows with 256 keys or more (decode shapes),
@@ -28,6 +33,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <cmath>
 
 #include "iak.h"
 #include "iak_device.h"
@@ -110,18 +117,20 @@ struct DenseSplit {
   int splits;   // workgroups per row
   int chunk;    // keys per workgroup (the last may have fewer)
   float* ws;    // splits > 1: [rows * splits] max, [rows * splits] denominator, [rows * splits, v_dim] context
+  int64_t accoff;   // offset of the contexts in ws (floats)
+  int log2;         // the maxima are in the exp2 domain
 };
 
 // T: element type of q, k, v and out; NPL: dims per lane (head_dim and v_dim
-// are at most 64 * NPL); KEYS keys per wave and step; WAVES waves per workgroup
+// are at most 64 * NPL); KEYS keys per wave and step; WAVES waves per workgroup.
+// `item` = row * splits + split, row = b * q_len + i; `items` of them in all.
 template <typename T, int NPL, int KEYS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const iak_dense_attention_args a,
-                                                                      const DenseSplit sp) {
+__device__ __forceinline__ void dense_row(const iak_dense_attention_args& a, const DenseSplit& sp, int64_t item,
+                                          int64_t items) {
   __shared__ float part_acc[WAVES][64 * NPL];
   __shared__ float part_m[WAVES], part_l[WAVES];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t item = blockIdx.x;   // row * splits + split, row = b * q_len + i
   const int64_t row = item / sp.splits;
   const int split = (int)(item - row * sp.splits);
   const int64_t b = row / a.q_len;
@@ -262,12 +271,11 @@ __global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const iak_d
   }
   if (sp.splits > 1) {
     // this range's partial: max, denominator and unnormalised context
-    const int64_t n = (int64_t)gridDim.x;
     if (threadIdx.x == 0) {
       sp.ws[item] = M;
-      sp.ws[n + item] = L;
+      sp.ws[items + item] = L;
     }
-    float* wacc = sp.ws + 2 * n + item * a.v_dim;
+    float* wacc = sp.ws + sp.accoff + item * a.v_dim;
     for (int d = threadIdx.x; d < a.v_dim; d += 64 * WAVES) {
       float A = 0.f;
 #pragma unroll
@@ -286,6 +294,14 @@ __global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const iak_d
     store_t<T>(a.out, ooff + d, M == NEG_INF ? empty : A / L);
   }
 }
+
+template <typename T, int NPL, int KEYS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const iak_dense_attention_args a,
+                                                                      const DenseSplit sp) {
+  dense_row<T, NPL, KEYS, WAVES>(a, sp, blockIdx.x, gridDim.x);
+}
+
+#include "dense_matrix.h"
 
 constexpr int MERGE_THREADS = 256;
 constexpr int MAX_SPLITS = 1024;
@@ -311,27 +327,36 @@ __device__ __forceinline__ float block_reduce(float v, float* red) {
 // (splits <= MAX_SPLITS). The split weights go to the LDS; each context dim is
 // then summed over the splits by G thread groups (G = 256 / dims rounded up to
 // 64), each over every G-th split, with eight independent loads in flight.
-template <typename T>
+// FLAGS: the partials come from dense_matrix_kernel with key-tile flags; a row of
+// a flagged batch entry is computed again from its inputs.
+template <typename T, bool FLAGS>
 __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const iak_dense_attention_args a,
-                                                                    const DenseSplit sp) {
+                                                                    const DenseSplit sp, const MatrixPlan mp) {
   __shared__ float wt[MAX_SPLITS];
   __shared__ float red[MERGE_THREADS / 64];
   __shared__ float part[MERGE_THREADS];
   const int64_t row = blockIdx.x;
   const int64_t b = row / a.q_len;
   const int i = (int)(row - b * a.q_len);
+  if constexpr (FLAGS) {
+    if (mx_flagged(mp, b)) {
+      dense_row<T, MX_MAX_DIM / 64, 2, MERGE_THREADS / 64>(a, DenseSplit{1, a.kv_len, nullptr, 0, 0}, row, 0);
+      return;
+    }
+  }
   const int S = sp.splits;
   const int64_t n = (int64_t)gridDim.x * S;
   const float* wm = sp.ws + row * S;
   const float* wl = sp.ws + n + row * S;
-  const float* wacc = sp.ws + 2 * n + row * S * a.v_dim;
+  const float* wacc = sp.ws + sp.accoff + row * S * a.v_dim;
   const float NEG_INF = -__builtin_inff();
   float mx = NEG_INF;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) mx = fmaxf(mx, wm[s]);
   const float M = block_reduce<true>(mx, red);
   float ls = 0.f;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) {
-    const float w = wm[s] == NEG_INF ? 0.f : expf(wm[s] - M);   // 0 for a range that saw no mass
+    // 0 for a range that saw no mass
+    const float w = wm[s] == NEG_INF ? 0.f : (sp.log2 ? __builtin_amdgcn_exp2f(wm[s] - M) : expf(wm[s] - M));
     wt[s] = w;
     ls += w * wl[s];
   }
@@ -387,7 +412,7 @@ void launch_items(const iak_dense_attention_args& a, const DenseSplit& sp, int64
 }
 
 template <typename T>
-void launch_typed(const iak_dense_attention_args& a, const DenseSplit& sp, hipStream_t stream) {
+void launch_rows(const iak_dense_attention_args& a, const DenseSplit& sp, hipStream_t stream) {
   const int64_t rows = (int64_t)a.batch * a.q_len;
   const int64_t items = rows * sp.splits;
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
@@ -398,7 +423,9 @@ void launch_typed(const iak_dense_attention_args& a, const DenseSplit& sp, hipSt
   else if (npl <= 4) launch_items<T, 4, 4, 16>(a, sp, items, stream);
   else if (npl <= 8) launch_items<T, 8, 4, 8>(a, sp, items, stream);
   else launch_items<T, 16, 2, 8>(a, sp, items, stream);
-  if (sp.splits > 1) hipLaunchKernelGGL(dense_merge_kernel<T>, dim3((unsigned)rows), dim3(256), 0, stream, a, sp);
+  if (sp.splits > 1)
+    hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp,
+                       MatrixPlan{});
 }
 
 // Splits per row: rows with SPLIT_MIN_KEYS keys or more on a short grid (fewer
@@ -406,7 +433,7 @@ void launch_typed(const iak_dense_attention_args& a, const DenseSplit& sp, hipSt
 // least RANGE_MIN_KEYS keys
 // (at most MAX_SPLITS ranges).
 DenseSplit split_plan(const iak_dense_attention_args& a) {
-  DenseSplit sp{1, a.kv_len, nullptr};
+  DenseSplit sp{1, a.kv_len, nullptr, 0, 0};
   const int64_t rows = (int64_t)a.batch * a.q_len;
   if (rows <= 0 || rows >= 512 || a.kv_len < SPLIT_MIN_KEYS) return sp;
   int64_t s = (SPLIT_TARGET_WGS + rows - 1) / rows;
@@ -417,24 +444,170 @@ DenseSplit split_plan(const iak_dense_attention_args& a) {
   const int64_t chunk = ((int64_t)a.kv_len + s - 1) / s;
   sp.splits = (int)(((int64_t)a.kv_len + chunk - 1) / chunk);
   sp.chunk = (int)chunk;
+  sp.accoff = 2 * rows * sp.splits;
   return sp;
+}
+
+// ---- the matrix-core form: which calls take it, and its plan ----
+
+// From this many (query, key) pairs on, and from this many query rows per batch
+// entry, the matrix form is the faster one (10 calls in a graph, us, rows form
+// against this one; 16-bit: 32 x 64 keys x 16 rows = 32,768 pairs 8.0 / 8.2 and
+// x 32 rows 10.5 / 8.3; 8 x 512 x 8 rows = 32,768 12.8 / 11.1; 8 x 4,096 x 2
+// rows 17.7 / 14.4; 32 x 4,096 x 32 rows 347 / 21; float32: 32 x 512 x 3 rows =
+// 49,152 22.9 / 18.3; 1 x 2,048 x 16 rows = 32,768 14.0 / 17.1; 8 x 4,096 x 2
+// rows 18.2 / 19.9). One query row keeps the rows form: equal at best.
+#ifndef MX_MIN_PAIRS
+#define MX_MIN_PAIRS 32768
+#define MX_MIN_PAIRS_F32 49152
+#define MX_MIN_ROWS 2
+#define MX_MIN_ROWS_F32 3
+#endif
+
+struct MatrixShape {
+  int dp;       // dims, padded
+  int qw, kw;   // waves over query rows and over keys
+  int bkw;      // keys per wave and tile
+};
+
+// 16-byte pieces of whole elements on every operand, at most 256 dims
+bool matrix_applies(const iak_dense_attention_args& a) {
+  const int es = a.dtype == IAK_DTYPE_F32 ? 4 : 2, vec = 16 / es;
+  const double pairs = (double)a.batch * a.q_len * a.kv_len;
+  if (a.q_len < (es == 4 ? MX_MIN_ROWS_F32 : MX_MIN_ROWS) || pairs < (es == 4 ? MX_MIN_PAIRS_F32 : MX_MIN_PAIRS)) return false;
+  const int most = es == 4 ? MX_MAX_DIM_F32 : MX_MAX_DIM;
+  if (a.head_dim > most || a.v_dim > most || a.head_dim % vec || a.v_dim % vec) return false;
+  if (!(a.sm_scale > 0.f) || !std::isfinite(a.sm_scale)) return false;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+                       reinterpret_cast<uintptr_t>(a.v);
+  if ((at & 15u) || (reinterpret_cast<uintptr_t>(a.out) & (4 * es - 1))) return false;
+  const int64_t row_strides = a.q_stride_t | a.k_stride_t | a.v_stride_t;
+  const int64_t batch_strides = a.batch > 1 ? (a.q_stride_b | a.k_stride_b | a.v_stride_b) : 0;
+  if ((row_strides | batch_strides) & (vec - 1)) return false;
+  if ((a.out_stride_t | (a.batch > 1 ? a.out_stride_b : 0)) & 3) return false;
+  return true;
+}
+
+MatrixShape matrix_shape(const iak_dense_attention_args& a) {
+  const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
+  MatrixShape s{64, 4, 1, 64};
+  const bool f32 = a.dtype == IAK_DTYPE_F32;
+  s.dp = width <= 64 ? 64 : (width <= 96 && !f32) ? 96 : width <= 128 ? 128 : width <= 192 ? 192 : 256;
+  if (f32) s.bkw = 32;
+  // few query rows: the four waves share out the keys instead
+  if (a.q_len <= 32 && s.dp <= 128) s.qw = 1, s.kw = 4, s.bkw = 32;
+  else if (a.q_len <= 64 && s.dp <= 128) s.qw = 2, s.kw = 2, s.bkw = 32;
+  return s;
+}
+
+// query tiles of 32 * qw rows; on short grids the keys go over about 256
+// workgroups in ranges of whole tiles
+MatrixPlan matrix_plan(const iak_dense_attention_args& a, const MatrixShape& s) {
+  MatrixPlan mp{};
+  const int64_t bq = 32 * s.qw, bk = s.kw * s.bkw;
+  mp.nq = (int)((a.q_len + bq - 1) / bq);
+  mp.nt = (int)((a.kv_len + bk - 1) / bk);
+  mp.skip = a.causal == IAK_CAUSAL_TRIU && !a.mask && a.sm_scale <= 1.f;
+  const int64_t wgs = (int64_t)a.batch * mp.nq;
+  int64_t n = wgs > 0 && wgs < SPLIT_TARGET_WGS ? SPLIT_TARGET_WGS / wgs : 1;
+  if (n > mp.nt) n = mp.nt;
+  if (n > MAX_SPLITS) n = MAX_SPLITS;
+  const int64_t per = ((int64_t)mp.nt + n - 1) / n;   // tiles per range
+  mp.splits = (int)((mp.nt + per - 1) / per);
+  mp.chunk = mp.splits > 1 ? (int)(per * bk) : a.kv_len;
+  mp.accoff = (2 * (int64_t)a.batch * a.q_len * mp.splits + 3) / 4 * 4;
+  return mp;
+}
+
+// key-tile flags are needed where a weight is split or tiles are skipped
+bool matrix_flags(const iak_dense_attention_args& a, const MatrixPlan& mp) {
+  return a.dtype != IAK_DTYPE_F32 || mp.skip;
+}
+
+size_t matrix_partial_bytes(const iak_dense_attention_args& a, const MatrixPlan& mp) {
+  if (mp.splits <= 1) return 0;
+  return ((size_t)mp.accoff + (size_t)a.batch * a.q_len * mp.splits * (size_t)a.v_dim) * sizeof(float);
+}
+
+size_t matrix_workspace(const iak_dense_attention_args& a) {
+  const MatrixPlan mp = matrix_plan(a, matrix_shape(a));
+  const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * 4 * sizeof(int32_t) : 0;
+  const size_t total = matrix_partial_bytes(a, mp) + flags;
+  return total ? total : 16;   // a workspace at all says that the form may run
+}
+
+template <typename T, int DP, int QW, int KW, int BKW>
+void launch_matrix_cfg(const iak_dense_attention_args& a, const MatrixPlan& mp, hipStream_t stream) {
+  const dim3 grid((unsigned)((int64_t)a.batch * mp.nq * mp.splits));
+  if (a.mask || a.causal == IAK_CAUSAL_POSITIONS)
+    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, true>), grid, dim3(MX_THREADS), 0, stream,
+                       a, mp);
+  else
+    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, false>), grid, dim3(MX_THREADS), 0, stream,
+                       a, mp);
+}
+
+template <typename T, int DP>
+void launch_matrix_dims(const iak_dense_attention_args& a, const MatrixShape& s, const MatrixPlan& mp,
+                        hipStream_t stream) {
+  constexpr int BKW = sizeof(T) == 4 ? 32 : 64;
+  if constexpr (DP <= 128) {
+    if (s.kw == 4) return launch_matrix_cfg<T, DP, 1, 4, 32>(a, mp, stream);
+    if (s.kw == 2) return launch_matrix_cfg<T, DP, 2, 2, 32>(a, mp, stream);
+  }
+  launch_matrix_cfg<T, DP, 4, 1, BKW>(a, mp, stream);
+}
+
+template <typename T>
+void launch_matrix(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
+  const MatrixShape s = matrix_shape(a);
+  MatrixPlan mp = matrix_plan(a, s);
+  mp.ws = static_cast<float*>(workspace);
+  const bool flags = matrix_flags(a, mp);
+  if (flags) mp.flags = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + matrix_partial_bytes(a, mp));
+  if (s.dp == 64) launch_matrix_dims<T, 64>(a, s, mp, stream);
+  else if (s.dp == 128) launch_matrix_dims<T, 128>(a, s, mp, stream);
+  if constexpr (sizeof(T) == 2) {
+    if (s.dp == 96) launch_matrix_dims<T, 96>(a, s, mp, stream);
+    else if (s.dp == 192) launch_matrix_dims<T, 192>(a, s, mp, stream);
+    else if (s.dp == 256) launch_matrix_dims<T, 256>(a, s, mp, stream);
+  }
+  const int64_t rows = (int64_t)a.batch * a.q_len;
+  if (mp.splits > 1) {
+    const bool gen = a.mask || a.causal == IAK_CAUSAL_POSITIONS;
+    const DenseSplit sp{mp.splits, mp.chunk, mp.ws, mp.accoff, gen ? 0 : 1};
+    if (flags)
+      hipLaunchKernelGGL((dense_merge_kernel<T, true>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
+    else
+      hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
+  } else if (flags) {
+    const int64_t per = a.batch < 256 ? (256 + a.batch - 1) / a.batch : 1;
+    hipLaunchKernelGGL(dense_fixup_kernel<T>, dim3((unsigned)(a.batch * per)), dim3(256), 0, stream, a, mp);
+  }
+}
+
+template <typename T>
+void launch_typed(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
+  if (workspace && matrix_applies(a)) return launch_matrix<T>(a, workspace, stream);
+  DenseSplit sp = split_plan(a);
+  if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr, 0, 0};
+  sp.ws = static_cast<float*>(workspace);
+  launch_rows<T>(a, sp, stream);
 }
 
 }  // namespace
 
 size_t dense_attention_workspace(const iak_dense_attention_args& a) {
   const DenseSplit sp = split_plan(a);
-  if (sp.splits <= 1) return 0;
-  return (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.v_dim) * sizeof(float);
+  const size_t rows = sp.splits <= 1 ? 0 : (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.v_dim) * sizeof(float);
+  const size_t matrix = matrix_applies(a) ? matrix_workspace(a) : 0;
+  return rows > matrix ? rows : matrix;
 }
 
 hipError_t launch_dense_attention(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
-  DenseSplit sp = split_plan(a);
-  if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr};
-  sp.ws = static_cast<float*>(workspace);
-  if (a.dtype == IAK_DTYPE_F32) launch_typed<float>(a, sp, stream);
-  else if (a.dtype == IAK_DTYPE_F16) launch_typed<_Float16>(a, sp, stream);
-  else launch_typed<bf16_bits>(a, sp, stream);
+  if (a.dtype == IAK_DTYPE_F32) launch_typed<float>(a, workspace, stream);
+  else if (a.dtype == IAK_DTYPE_F16) launch_typed<_Float16>(a, workspace, stream);
+  else launch_typed<bf16_bits>(a, workspace, stream);
   return hipGetLastError();
 }
 

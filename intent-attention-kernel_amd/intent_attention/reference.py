@@ -133,8 +133,8 @@ def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
         if positions is not None:
             a.kv_positions = positions.data_ptr()
     a.sm_scale = 1.0 / math.sqrt(D)
-    # few rows with many keys: a workspace lets the kernel split each row's keys
-    # over several workgroups (decode shapes); the operands, any copies made
+    # a workspace lets the library run several query rows per batch entry on the
+    # matrix cores, and split few rows' keys over several workgroups; the operands, any copies made
     # above and the workspace were allocated on this stream, so the caching
     # allocator reuses their memory only after these kernels
     ws_bytes = N.dense_attention_workspace(a)

@@ -1,0 +1,129 @@
+"""dense_attention on the matrix-core form (csrc/dense_matrix.h): the edges of its
+query and key tiles, padded widths, every mask form, strided and broadcast operands,
+and non-finite values, against the float64 oracle and against the row form (the
+library without a workspace), which the form has to agree with value for value up
+to rounding and NaN / infinity for NaN / infinity."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import attention as A
+
+pytestmark = pytest.mark.gpu
+
+DT = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+# float32: 2e-5 as elsewhere for float32 sums; 16-bit outputs: half an ulp of values
+# of at most 4 besides (2^-10 and 2^-7 relative spacing halves)
+TOL = {"f16": 2e-5 + 4 * 2 ** -11, "bf16": 2e-5 + 4 * 2 ** -8, "f32": 2e-5}
+
+
+def _rows_form(monkeypatch, *a, **kw):
+    from intent_attention import _native as N
+    from intent_attention import dense_attention
+    with monkeypatch.context() as mp:
+        mp.setattr(N, "dense_attention_workspace", lambda args: 0)
+        return dense_attention(*a, **kw)
+
+
+def _qkv(seed, lead, tq, tk, d, dv, dt):
+    g = torch.Generator().manual_seed(seed)
+    mk = lambda *s: torch.randn(*s, generator=g).to(DT[dt])  # noqa: E731
+    return mk(*lead, tq, d), mk(*lead, tk, d), mk(*lead, tk, dv), g
+
+
+def _check(got, want, dt, what):
+    o = got.double().cpu().numpy()
+    err = np.abs(o - want).max()
+    print(f"[gpu-case] {what}: max abs err {err:.2e}", flush=True)
+    assert err <= TOL[dt], what
+
+
+# (tq, tk, d, dv): one below, at and one above the query tiles (32, 64, 128 rows) and the
+# key tiles (64 or 128 keys), the smallest widths, padded ones, unequal ones, the widest
+SHAPES = [(31, 64, 64, 64), (32, 65, 64, 64), (33, 63, 128, 128), (64, 129, 128, 64), (65, 127, 64, 128),
+          (127, 300, 128, 128), (128, 1, 64, 64), (129, 513, 96, 96), (257, 257, 72, 80), (40, 200, 8, 16),
+          (100, 130, 192, 136), (70, 190, 256, 200), (2, 1500, 128, 128), (5, 700, 64, 64)]
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("tq,tk,d,dv", SHAPES)
+def test_tile_edges(tq, tk, d, dv, dt):
+    from intent_attention import dense_attention
+    lead = (2, max(2, -(-50000 // (2 * tq * tk))))
+    q, k, v, _ = _qkv(tq * 1000 + tk, lead, tq, tk, d, dv, dt)
+    n = lambda *x: [t.double().numpy() for t in x]  # noqa: E731
+    c = lambda *x: [t.cuda() for t in x]  # noqa: E731
+    for causal in (False, True):
+        _check(dense_attention(*c(q, k, v), causal=causal), A.dense_attention_masked(*n(q, k, v), causal=causal), dt,
+               f"{dt} {lead} {tq}x{tk}x{d}/{dv} causal={causal}")
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("tq,tk", [(12, 900), (130, 200)])
+def test_masks_positions_and_layouts(tq, tk, dt, monkeypatch):
+    from intent_attention import dense_attention
+    q, k, v, g = _qkv(7, (2, 4), tq, tk, 64, 64, dt)
+    mask = torch.randn(tq, tk, generator=g)
+    mask[torch.rand(tq, tk, generator=g) < 0.3] = float("-inf")
+    mask[:, 3] = 0.0
+    low = torch.zeros(tq, tk).to(DT[dt])
+    low[:, tk // 2:] = torch.finfo(DT[dt]).min
+    low[1] = torch.finfo(DT[dt]).min            # a whole row of the lowest value: still a softmax
+    dead = torch.zeros(tq, tk).to(DT[dt])
+    dead[2] = float("-inf")                     # a row with nothing to attend: NaN
+    pos = torch.sort(torch.randperm(3 * tk, generator=g)[:tk]).values
+    pos[0] = 0
+    bools = torch.rand(2, 1, tq, tk, generator=g) < 0.5
+    cases = [dict(mask=mask.to(DT[dt])), dict(mask=low), dict(mask=dead), dict(mask=bools),
+             dict(causal=True, mask=mask.to(DT[dt])), dict(causal=True, original_kv_positions=pos),
+             dict(causal=True, original_kv_positions=pos.flip(0))]
+    qc, kc, vc = q.cuda(), k.cuda(), v.cuda()
+    # [B, T, H, D] storage, and K / V broadcast over the heads
+    swapped = [x.transpose(1, 2).contiguous().transpose(1, 2) for x in (qc, kc, vc)]
+    shared = [qc, kc[:, :1], vc[:, :1]]
+    for kw in cases:
+        kw = {n: (x.cuda() if isinstance(x, torch.Tensor) else x) for n, x in kw.items()}
+        for ops in ((qc, kc, vc), swapped, shared):
+            got, want = dense_attention(*ops, **kw), _rows_form(monkeypatch, *ops, **kw)
+            assert torch.equal(torch.isnan(got), torch.isnan(want)), sorted(kw)
+            live = ~torch.isnan(want)
+            assert float((got[live].double() - want[live].double()).abs().max()) <= 2 * TOL[dt], sorted(kw)
+
+
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("tq,tk,d", [(128, 300, 64), (300, 300, 128), (16, 2200, 64), (1100, 700, 64)])
+def test_nonfinite_values_as_the_row_form(tq, tk, d, dt, monkeypatch):
+    """Infinities, NaN and values whose scores overflow, in visible and in causally hidden
+    keys, give what the plain sums give: the tiles past the diagonal and the split of
+    the weights must not hide or invent one."""
+    from intent_attention import dense_attention
+    big = 60000.0 if dt == "f16" else 1e37
+    for where, value in (("k", np.inf), ("k", np.nan), ("v", np.inf), ("v", -np.inf), ("v", np.nan), ("k", big),
+                         ("q", np.inf), ("q", big)):
+        for causal in (False, True):
+            q, k, v, _ = _qkv(11, (1, 2), tq, tk, d, d, dt)
+            x, at = {"q": (q, tq // 2), "k": (k, tk - 5), "v": (v, tk - 5)}[where]
+            x[0, 0, at, 3 if abs(value) != big else slice(None)] = value
+            ops = [t.cuda() for t in (q, k, v)]
+            got, want = dense_attention(*ops, causal=causal), _rows_form(monkeypatch, *ops, causal=causal)
+            what = f"{where}={value} causal={causal}"
+            assert torch.equal(torch.isnan(got), torch.isnan(want)), what
+            assert torch.equal(torch.isinf(got), torch.isinf(want)), what
+            live = torch.isfinite(want)
+            assert float((got[live].double() - want[live].double()).abs().max()) <= 2 * TOL[dt], what
+
+
+def test_replays_from_a_graph():
+    from intent_attention import dense_attention
+    q, k, v, g = _qkv(3, (1, 8), 200, 333, 128, 128, "f16")
+    qc, kc, vc = q.cuda(), k.cuda(), v.cuda()
+    eager = dense_attention(qc, kc, vc, causal=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = dense_attention(qc, kc, vc, causal=True)
+    for i in range(3):
+        qc.copy_(torch.randn(q.shape, generator=g).half())
+        graph.replay()
+        want = dense_attention(qc, kc, vc, causal=True)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and not torch.equal(out, eager), i
