@@ -21,6 +21,9 @@
 // past the end of C (the last page's missing rows) takes no mass. A latent row
 // is both the key and the value of its token, so it is loaded once.
 //
+// Calls with several query rows run on the matrix cores (mla_rows_matrix.h); what
+// follows is the rows form, for the rest.
+//
 // Work split. Every query row attends to the same latent rows, so a
 // workgroup takes four query rows once there are four (each latent row it
 // loads serves all of them). A row group's keys go to `splits` workgroups of
@@ -38,6 +41,8 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 #include "iak.h"
 #include "iak_device.h"
@@ -96,6 +101,8 @@ struct RowSplit {
   uint32_t magic;    // floor(2^32 / page_size), or 2^32 - 1 for page_size 1
   int rows_per_wg;   // query rows per workgroup (1 or 4)
   float* ws;         // splits > 1: [n] max, [n] denominator, [n, d_c] context, n = rows * splits
+  int64_t accoff;    // offset of the contexts in ws (floats)
+  int log2;          // the maxima are in the exp2 domain
 };
 
 // The C row of key j: outside [0, num_rows) for a key past the end of C or of
@@ -248,7 +255,7 @@ __global__ __launch_bounds__(64 * WAVES) void mla_rows_kernel(const iak_mla_rows
         sp.ws[slot] = M;
         sp.ws[n + slot] = L;
       }
-      float* wacc = sp.ws + 2 * n + slot * dc;
+      float* wacc = sp.ws + sp.accoff + slot * dc;
       for (int d = threadIdx.x; d < dc; d += 64 * WAVES) {
         float A = 0.f;
 #pragma unroll
@@ -287,63 +294,55 @@ __device__ __forceinline__ float block_reduce(float v, float* red) {
   return v;
 }
 
-// One workgroup per row: the log-sum-exp merge of the row's `splits` partials
-// (splits <= MAX_SPLITS), split weights in the LDS, each context dim summed
-// over the splits by G thread groups with eight loads in flight.
+// The log-sum-exp merge of a row's `splits` partials (splits <= MAX_SPLITS): one
+// workgroup per row and 64 dims, wave w over every fourth split with eight loads
+// in flight; the split weights are in the LDS, the waves meet there too. (One
+// workgroup per row left 32 rows on 32 CUs: 256 splits x 576 dims 8.5 us.)
 __global__ __launch_bounds__(MERGE_THREADS) void mla_rows_merge_kernel(const iak_mla_rows_args a,
                                                                        const RowSplit sp) {
+  constexpr int WAVES = MERGE_THREADS / 64;
   __shared__ float wt[MAX_SPLITS];
-  __shared__ float red[MERGE_THREADS / 64];
-  __shared__ float part[MERGE_THREADS];
+  __shared__ float red[WAVES];
+  __shared__ float part[WAVES][64];
   const int64_t row = blockIdx.x;
   const int S = sp.splits, dc = a.latent_dim;
   const int64_t n = (int64_t)gridDim.x * S;
   const float* wm = sp.ws + row * S;
   const float* wl = sp.ws + n + row * S;
-  const float* wacc = sp.ws + 2 * n + row * S * dc;
   const float NEG_INF = -__builtin_inff();
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int d = blockIdx.y * 64 + lane, dcl = d < dc ? d : dc - 1;
+  const float* wacc = sp.ws + sp.accoff + row * S * dc + dcl;
   float mx = NEG_INF;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) mx = fmaxf(mx, wm[s]);
   const float M = block_reduce<true>(mx, red);
   float ls = 0.f;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) {
-    const float w = wm[s] == NEG_INF ? 0.f : expf(wm[s] - M);   // 0 for a range that visited no row
-    wt[s] = w;
-    ls += w * wl[s];
+    // 0 for a range that visited no row
+    const float x = wm[s] == NEG_INF ? 0.f : (sp.log2 ? __builtin_amdgcn_exp2f(wm[s] - M) : expf(wm[s] - M));
+    wt[s] = x;
+    ls += x * wl[s];
   }
   const float L = block_reduce<false>(ls, red);   // its barriers also publish wt[]
-  const int dims = (dc + 63) & ~63;
-  const int G = dims >= MERGE_THREADS ? 1 : MERGE_THREADS / dims;
-  const int g = threadIdx.x / dims, dl = threadIdx.x - g * dims;
-  float* out = a.context + row * dc;
-  for (int d0 = 0; d0 < dc; d0 += MERGE_THREADS) {
-    const int d = d0 + (G > 1 ? dl : threadIdx.x);
-    const int dcl = d < dc ? d : dc - 1;
-    float A = 0.f;
-    if (g < G) {
-      int s = g;
-      for (; s + 7 * G < S; s += 8 * G) {
-        float x[8];
+  float A = 0.f;
+  int s = w;
+  for (; s + 7 * WAVES < S; s += 8 * WAVES) {
+    float x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = wacc[(int64_t)(s + u * G) * dc + dcl];
+    for (int u = 0; u < 8; ++u) x[u] = wacc[(int64_t)(s + u * WAVES) * dc];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) A = __builtin_fmaf(wt[s + u * G], x[u], A);
-      }
-      for (; s < S; s += G) A = __builtin_fmaf(wt[s], wacc[(int64_t)s * dc + dcl], A);
-    }
-    if (G > 1) {
-      // the G groups' sums of one dim: group 0 adds them in group order
-      part[threadIdx.x] = A;
-      __syncthreads();
-      if (g == 0) {
-        for (int k = 1; k < G; ++k) A += part[k * dims + dl];
-      }
-      __syncthreads();
-      if (g != 0) continue;
-    }
-    if (d < dc) out[d] = L > 0.f ? A / L : 0.f;
+    for (int u = 0; u < 8; ++u) A = __builtin_fmaf(wt[s + u * WAVES], x[u], A);
+  }
+  for (; s < S; s += WAVES) A = __builtin_fmaf(wt[s], wacc[(int64_t)s * dc], A);
+  part[w][lane] = A;
+  __syncthreads();
+  if (w == 0 && d < dc) {
+    A = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    a.context[row * dc + d] = L > 0.f ? A / L : 0.f;
   }
 }
+
+#include "mla_rows_matrix.h"
 
 // MAXW: the most waves per workgroup whose registers and LDS fit
 template <typename T, int NPL, int KEYS, int MAXW, int R>
@@ -375,10 +374,22 @@ void launch_rows(const iak_mla_rows_args& a, const RowSplit& sp, hipStream_t str
 template <typename T>
 void launch_typed(const iak_mla_rows_args& a, const RowSplit& sp, hipStream_t stream) {
   const int64_t rows = (int64_t)a.batch * a.q_len;
-  if (sp.rows_per_wg == 4) launch_rows<T, 4>(a, sp, stream);
-  else launch_rows<T, 1>(a, sp, stream);
+  if (sp.rows_per_wg == RX_ROWS) {
+    const dim3 grid((unsigned)((rows + RX_ROWS - 1) / RX_ROWS * sp.splits));
+    const int nd = rx_dim_tiles(a.latent_dim), waves = (a.latent_dim + 32 * nd - 1) / (32 * nd);
+    const dim3 block(64 * waves);
+    if (nd == 1 && waves <= 4) hipLaunchKernelGGL((mla_rows_matrix_kernel<T, 1, 4>), grid, block, 0, stream, a, sp);
+    else if (nd == 1) hipLaunchKernelGGL((mla_rows_matrix_kernel<T, 1, 8>), grid, block, 0, stream, a, sp);
+    else if (nd == 2) hipLaunchKernelGGL((mla_rows_matrix_kernel<T, 2, 8>), grid, block, 0, stream, a, sp);
+    else hipLaunchKernelGGL((mla_rows_matrix_kernel<T, 3, 8>), grid, block, 0, stream, a, sp);
+  } else if (sp.rows_per_wg == 4) {
+    launch_rows<T, 4>(a, sp, stream);
+  } else {
+    launch_rows<T, 1>(a, sp, stream);
+  }
   if (sp.splits > 1)
-    hipLaunchKernelGGL(mla_rows_merge_kernel, dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp);
+    hipLaunchKernelGGL(mla_rows_merge_kernel, dim3((unsigned)rows, (unsigned)((a.latent_dim + 63) / 64)),
+                       dim3(MERGE_THREADS), 0, stream, a, sp);
 }
 
 // Splits per row group: with fewer than 512 groups and SPLIT_MIN_KEYS keys or
@@ -389,7 +400,7 @@ void launch_typed(const iak_mla_rows_args& a, const RowSplit& sp, hipStream_t st
 // parallelism).
 RowSplit plan_for(const iak_mla_rows_args& a, int R) {
   const int64_t nkeys = (int64_t)a.num_selected * a.page_size;
-  RowSplit sp{1, (int)nkeys, (int)nkeys, 0u, R, nullptr};
+  RowSplit sp{1, (int)nkeys, (int)nkeys, 0u, R, nullptr, 0, 0};
   sp.magic = a.page_size == 1 ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / (uint64_t)a.page_size);
   const int64_t rows = (int64_t)a.batch * a.q_len;
   const int64_t groups = (rows + R - 1) / R;
@@ -402,10 +413,56 @@ RowSplit plan_for(const iak_mla_rows_args& a, int R) {
   const int64_t chunk = (nkeys + s - 1) / s;
   sp.splits = (int)((nkeys + chunk - 1) / chunk);
   sp.chunk = (int)chunk;
+  sp.accoff = 2 * rows * sp.splits;
+  return sp;
+}
+
+// From this many query rows and (row, key) pairs on the matrix form is the faster
+// one, by the 32-dim tiles a wave of it holds (its chain grows with them). Both
+// forms, us per call (float16 latents, 30 calls): 128 dims 4 x 8,192 22.5 / 12.3,
+// 16 x 2,048 21.9 / 10.0; 512 dims 32 x 512 = 16,384 12.9 / 16.7, 16 x 2,048 =
+// 32,768 21.1 / 16.6, 4 x 8,192 21.9 / 18.9; 576 dims 8 x 8,192 = 65,536 22.9 /
+// 25.0, 64 x 2,048 30.4 / 25.0, 16 x 8,192 = 131,072 29.7 / 26.5, 32 x 8,192
+// 43.8 / 28.9 (52 before the merge went over the dims as well).
+#ifndef RX_MIN_ROWS
+#define RX_MIN_ROWS 4
+#endif
+#ifdef RX_MIN_PAIRS
+constexpr double rx_min_pairs(int) { return RX_MIN_PAIRS; }
+#else
+constexpr double rx_min_pairs(int nd) { return nd == 1 ? 2048 : nd == 2 ? 32768 : 131072; }
+#endif
+
+// whole 16-byte pieces of every latent row, at most 768 dims
+bool matrix_applies(const iak_mla_rows_args& a) {
+  const int vec = a.latent_dtype == IAK_DTYPE_F32 ? 4 : 8;
+  const int64_t rows = (int64_t)a.batch * a.q_len, nkeys = (int64_t)a.num_selected * a.page_size;
+  return rows >= RX_MIN_ROWS && nkeys > 0 && (double)rows * nkeys >= rx_min_pairs(rx_dim_tiles(a.latent_dim)) && a.num_rows > 0 &&
+         rx_dim_tiles(a.latent_dim) <= RX_MAX_ND && a.latent_dim % vec == 0 && a.sm_scale > 0.f &&
+         !((reinterpret_cast<uintptr_t>(a.latents) | reinterpret_cast<uintptr_t>(a.context)) & 15u) &&
+         a.latent_stride % vec == 0;
+}
+
+// 32 query rows per workgroup, the keys over about 256 workgroups in ranges of
+// whole 32-key tiles
+RowSplit matrix_plan(const iak_mla_rows_args& a) {
+  const int64_t nkeys = (int64_t)a.num_selected * a.page_size, rows = (int64_t)a.batch * a.q_len;
+  RowSplit sp{1, (int)nkeys, (int)nkeys, 0u, RX_ROWS, nullptr, 0, 1};
+  sp.magic = a.page_size == 1 ? 0xFFFFFFFFu : (uint32_t)((1ull << 32) / (uint64_t)a.page_size);
+  const int64_t groups = (rows + RX_ROWS - 1) / RX_ROWS, tiles = (nkeys + RX_KEYS - 1) / RX_KEYS;
+  int64_t s = groups < SPLIT_TARGET_WGS ? SPLIT_TARGET_WGS / groups : 1;
+  if (s > tiles) s = tiles;
+  if (s > MAX_SPLITS) s = MAX_SPLITS;
+  if (s <= 1) return sp;
+  const int64_t per = (tiles + s - 1) / s;
+  sp.splits = (int)((tiles + per - 1) / per);
+  sp.chunk = sp.splits > 1 ? (int)(per * RX_KEYS) : (int)nkeys;
+  sp.accoff = (2 * rows * sp.splits + 3) / 4 * 4;
   return sp;
 }
 
 RowSplit split_plan(const iak_mla_rows_args& a) {
+  if (matrix_applies(a)) return matrix_plan(a);
   const int64_t rows = (int64_t)a.batch * a.q_len;
   if (rows >= 4) {
     const RowSplit sp4 = plan_for(a, 4);
@@ -419,7 +476,7 @@ RowSplit split_plan(const iak_mla_rows_args& a) {
 size_t mla_rows_workspace(const iak_mla_rows_args& a) {
   const RowSplit sp = split_plan(a);
   if (sp.splits <= 1) return 0;
-  return (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.latent_dim) * sizeof(float);
+  return ((size_t)sp.accoff + (size_t)a.batch * a.q_len * sp.splits * (size_t)a.latent_dim) * sizeof(float);
 }
 
 hipError_t launch_mla_rows(const iak_mla_rows_args& a, void* workspace, hipStream_t stream) {
