@@ -226,8 +226,24 @@ iak_status validate(const iak_paged_decode_args* a, Plan* plan, bool tiers = tru
   return IAK_OK;
 }
 
+// The few-heads MLA form is taken for at most 16 heads, unless they read FP8 / INT8
+// latents of 512 dims or more (which each wave then converts for itself), and for
+// more heads over one or two short tables, where its workgroups per 16 heads use
+// more of the chip. Both forms, us per call (split kernel and merge): 16 heads x
+// 576 dims, float16, 8 x 300 pages 28.5 / 25.1, 32 x 512 99.0 / 77.7; FP8 / INT8
+// 8 x 300 24.6 / 26.4; 8 heads 23.9 / 23.8; 16 heads x 128 dims 8 x 300 14.6 /
+// 12.2, 32 x 512 44.6 / 34.0; 1 x 512 pages, 64 heads x 576 34.7 / 24.1; 8 x 300,
+// 32 heads x 576 30.5 / 30.1, 64 heads 35.1 / 42.8.
+constexpr long long MLA_FEW_VISITS = 4096;   // pages x groups of 16 heads
+bool mla_few_heads(const iak_mla_decode_args* a, bool fp16) {
+  if (a->num_heads <= 16 && (a->num_heads <= 8 || fp16 || a->qk_dim <= 256)) return true;
+  return a->num_heads > 16 && a->batch <= 2 &&
+         (long long)a->batch * a->table_width * ((a->num_heads + 15) / 16) <= MLA_FEW_VISITS;
+}
+
 struct MPlan {
   int splits, chunk, HG;
+  bool few;
   size_t ws_m, ws_l, ws_acc, total;
 };
 
@@ -262,11 +278,12 @@ iak_status validate_mla(const iak_mla_decode_args* a, MPlan* plan) {
     if (!a->page_table || !a->page_counts) return fail(IAK_EINVAL, "page_table/page_counts is NULL");
   }
   // latent pools reachable through the tag map (no tags: every page FP16)
+  bool fp16 = false;
   for (int t = 0; t < 8; ++t) {
     const int n = a->page_tags ? a->tag_map[t] : (t == 0 ? IAK_TAG_FP16 : IAK_TAG_SKIP);
     const void *pool = nullptr, *sc = nullptr;
     switch (n) {
-      case IAK_TAG_FP16: pool = a->c_fp16; sc = pool; break;
+      case IAK_TAG_FP16: pool = a->c_fp16; sc = pool; fp16 = true; break;
       case IAK_TAG_FP8: pool = a->c_fp8; sc = a->c_fp8_scale; break;
       case IAK_TAG_INT8: pool = a->c_int8; sc = a->c_int8_scale; break;
       case IAK_TAG_INT4:
@@ -278,15 +295,18 @@ iak_status validate_mla(const iak_mla_decode_args* a, MPlan* plan) {
     if (!aligned16(pool)) return fail(IAK_EINVAL, "%s latent pool must be 16-byte aligned", tag_name(n));
   }
 
-  // split plan: one workgroup per (sequence, split, 128 heads); enough
-  // workgroups for every CU when the table is long enough
+  // split plan: one workgroup per (sequence, split, 128 heads), or 16 heads in the
+  // few-heads form; enough workgroups for every CU when the table is long enough
   const int W = a->table_width;
-  const int HG = (a->num_heads + 127) / 128;
+  const bool few = mla_few_heads(a, fp16);
+  const int HG = few ? (a->num_heads + 15) / 16 : (a->num_heads + 127) / 128;
   int chunk = a->pages_per_split;
   if (chunk == 0) {
     const long long units = (long long)a->batch * HG;
-    const long long want = units > 0 ? (256 + units - 1) / units : 1;
-    chunk = (int)((W + want - 1) / (want > 0 ? want : 1));
+    // (few heads: one workgroup per CU fits, so no more than 256 of them)
+    const long long want = units > 0 ? (few ? 256 / units : (256 + units - 1) / units) : 1;
+    chunk = (int)((W + (want > 0 ? want : 1) - 1) / (want > 0 ? want : 1));
+    if (few && chunk < 4) chunk = 4;   // a page for each wave
     if (chunk > 128) chunk = 128;
     if (chunk < 1) chunk = 1;
   }
@@ -296,6 +316,7 @@ iak_status validate_mla(const iak_mla_decode_args* a, MPlan* plan) {
   plan->splits = splits;
   plan->chunk = chunk;
   plan->HG = HG;
+  plan->few = few;
   if (splits == 1) {
     plan->ws_m = plan->ws_l = plan->ws_acc = plan->total = 0;
   } else {
@@ -581,7 +602,7 @@ static iak_status mla_decode_impl(const iak_mla_decode_args* a, void* workspace,
   std::memset(&m, 0, sizeof(m));
   m.B = a->batch; m.H = a->num_heads; m.DQK = a->qk_dim; m.DV = a->v_dim; m.VOFF = a->v_offset;
   m.W = a->table_width; m.NP = a->num_pages;
-  m.splits = plan.splits; m.chunk = plan.chunk; m.HG = plan.HG;
+  m.splits = plan.splits; m.chunk = plan.chunk; m.HG = plan.HG; m.few = plan.few;
   m.q = a->q; m.q_dtype = a->q_dtype; m.qsb = a->q_stride_b; m.qsh = a->q_stride_h;
   m.out = a->out; m.out_dtype = a->out_dtype; m.osb = a->out_stride_b; m.osh = a->out_stride_h;
   m.table = a->page_table; m.counts = a->page_counts; m.tags = a->page_tags;

@@ -495,11 +495,16 @@ __global__ __launch_bounds__(512, 1) void mla_decode_kernel(const MArgs a) {
   }
 }
 
+#include "mla_few.h"
+
 template <int DQK, int DV, bool WIDE>
 hipError_t launch_mla_w(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
   if (ev_begin) (void)hipEventRecord(ev_begin, stream);
-  hipLaunchKernelGGL((mla_decode_kernel<DQK, DV, WIDE>), dim3(m.B * m.splits, m.HG),
-                     dim3(Mla<DQK, DV, WIDE>::THREADS), 0, stream, m);
+  if (m.few)
+    hipLaunchKernelGGL((mla_few_heads_kernel<DQK, DV>), dim3(m.B * m.splits, m.HG), dim3(64 * FEW_WAVES), 0, stream, m);
+  else
+    hipLaunchKernelGGL((mla_decode_kernel<DQK, DV, WIDE>), dim3(m.B * m.splits, m.HG),
+                       dim3(Mla<DQK, DV, WIDE>::THREADS), 0, stream, m);
   hipError_t e = hipGetLastError();
   if (ev_end) (void)hipEventRecord(ev_end, stream);
   if (e != hipSuccess || m.splits == 1) return e;
