@@ -369,6 +369,7 @@ iak_status scratch_address(int dev, void** out) {
 
 namespace iak {
 hipError_t launch_mla_rows(const iak_mla_rows_args& a, void* workspace, hipStream_t stream);   // mla_rows.hip
+hipError_t launch_mla_few_heads(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end);   // mla_decode.hip; HG = groups of 16 heads
 size_t mla_rows_workspace(const iak_mla_rows_args& a);                                      // mla_rows.hip
 hipError_t launch_fake_quant_blocks(const iak_fake_quant_blocks_args& a, void* workspace,
                                     hipStream_t stream);                    // fake_quant.hip
@@ -602,7 +603,7 @@ static iak_status mla_decode_impl(const iak_mla_decode_args* a, void* workspace,
   std::memset(&m, 0, sizeof(m));
   m.B = a->batch; m.H = a->num_heads; m.DQK = a->qk_dim; m.DV = a->v_dim; m.VOFF = a->v_offset;
   m.W = a->table_width; m.NP = a->num_pages;
-  m.splits = plan.splits; m.chunk = plan.chunk; m.HG = plan.HG; m.few = plan.few;
+  m.splits = plan.splits; m.chunk = plan.chunk; m.HG = plan.HG;
   m.q = a->q; m.q_dtype = a->q_dtype; m.qsb = a->q_stride_b; m.qsh = a->q_stride_h;
   m.out = a->out; m.out_dtype = a->out_dtype; m.osb = a->out_stride_b; m.osh = a->out_stride_h;
   m.table = a->page_table; m.counts = a->page_counts; m.tags = a->page_tags;
@@ -633,8 +634,8 @@ static iak_status mla_decode_impl(const iak_mla_decode_args* a, void* workspace,
     m.ws_l = reinterpret_cast<float*>(ws + plan.ws_l);
     m.ws_acc = reinterpret_cast<float*>(ws + plan.ws_acc);
   }
-  const hipError_t e = iak::launch_mla_decode(m, static_cast<hipStream_t>(stream),
-                                              static_cast<hipEvent_t>(ev_begin), static_cast<hipEvent_t>(ev_end));
+  const hipError_t e = (plan.few ? iak::launch_mla_few_heads : iak::launch_mla_decode)(
+      m, static_cast<hipStream_t>(stream), static_cast<hipEvent_t>(ev_begin), static_cast<hipEvent_t>(ev_end));
   if (e != hipSuccess) return fail(IAK_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
   return IAK_OK;
 }

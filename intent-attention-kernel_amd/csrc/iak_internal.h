@@ -98,8 +98,7 @@ struct MArgs {
   int64_t NP;
   int splits;   // splits per sequence
   int chunk;    // table entries per split (<= 128)
-  int HG;       // groups of 128 heads (few: of 16)
-  int few;      // the few-heads form: a workgroup's waves share out the pages
+  int HG;       // groups of 128 heads
 
   const void* q; int q_dtype; int64_t qsb, qsh;
   void* out; int out_dtype; int64_t osb, osh;

@@ -497,23 +497,32 @@ __global__ __launch_bounds__(512, 1) void mla_decode_kernel(const MArgs a) {
 
 #include "mla_few.h"
 
-template <int DQK, int DV, bool WIDE>
-hipError_t launch_mla_w(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
-  if (ev_begin) (void)hipEventRecord(ev_begin, stream);
-  if (m.few)
-    hipLaunchKernelGGL((mla_few_heads_kernel<DQK, DV>), dim3(m.B * m.splits, m.HG), dim3(64 * FEW_WAVES), 0, stream, m);
-  else
-    hipLaunchKernelGGL((mla_decode_kernel<DQK, DV, WIDE>), dim3(m.B * m.splits, m.HG),
-                       dim3(Mla<DQK, DV, WIDE>::THREADS), 0, stream, m);
-  hipError_t e = hipGetLastError();
-  if (ev_end) (void)hipEventRecord(ev_end, stream);
-  if (e != hipSuccess || m.splits == 1) return e;
-  // the paged-decode merge over rows (b, 0) of H heads
+// the paged-decode merge over rows (b, 0) of H heads
+template <int DV> hipError_t launch_mla_merge(const MArgs& m, hipStream_t stream) {
   KArgs k{};
   k.B = m.B; k.Hq = m.H; k.Hkv = 1; k.G = m.H; k.D = DV; k.splits = m.splits;
   k.out = m.out; k.out_dtype = m.out_dtype; k.osb = m.osb; k.osh = m.osh;
   k.ws_m = m.ws_m; k.ws_l = m.ws_l; k.ws_acc = m.ws_acc; k.acc16 = m.acc16;
   return launch_merge<DV>(k, stream);
+}
+
+template <int DQK, int DV, bool WIDE>
+hipError_t launch_mla_w(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
+  if (ev_begin) (void)hipEventRecord(ev_begin, stream);
+  hipLaunchKernelGGL((mla_decode_kernel<DQK, DV, WIDE>), dim3(m.B * m.splits, m.HG),
+                     dim3(Mla<DQK, DV, WIDE>::THREADS), 0, stream, m);
+  const hipError_t e = hipGetLastError();
+  if (ev_end) (void)hipEventRecord(ev_end, stream);
+  return e != hipSuccess || m.splits == 1 ? e : launch_mla_merge<DV>(m, stream);
+}
+
+template <int DQK, int DV>
+hipError_t launch_few(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end) {
+  if (ev_begin) (void)hipEventRecord(ev_begin, stream);
+  hipLaunchKernelGGL((mla_few_heads_kernel<DQK, DV>), dim3(m.B * m.splits, m.HG), dim3(64 * FEW_WAVES), 0, stream, m);
+  const hipError_t e = hipGetLastError();
+  if (ev_end) (void)hipEventRecord(ev_end, stream);
+  return e != hipSuccess || m.splits == 1 ? e : launch_mla_merge<DV>(m, stream);
 }
 
 // WIDE: FP16 latent pages are reachable (ring slots sized for two bytes per value)
@@ -530,6 +539,19 @@ hipError_t launch_mla_decode(const MArgs& m, hipStream_t stream, hipEvent_t eb, 
     case 512512: return launch_mla<512, 512>(m, stream, eb, ee);
     case 576512: return launch_mla<576, 512>(m, stream, eb, ee);
     case 576064: return launch_mla<576, 64>(m, stream, eb, ee);
+  }
+  return hipErrorInvalidValue;
+}
+
+// the few-heads form (mla_few.h); m.HG counts groups of 16 heads
+hipError_t launch_mla_few_heads(const MArgs& m, hipStream_t stream, hipEvent_t eb, hipEvent_t ee) {
+  switch (m.DQK * 1000 + m.DV) {
+    case 64064: return launch_few<64, 64>(m, stream, eb, ee);
+    case 128128: return launch_few<128, 128>(m, stream, eb, ee);
+    case 256256: return launch_few<256, 256>(m, stream, eb, ee);
+    case 512512: return launch_few<512, 512>(m, stream, eb, ee);
+    case 576512: return launch_few<576, 512>(m, stream, eb, ee);
+    case 576064: return launch_few<576, 64>(m, stream, eb, ee);
   }
   return hipErrorInvalidValue;
 }
