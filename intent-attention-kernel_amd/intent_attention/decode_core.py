@@ -91,6 +91,13 @@ def current_stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def uploads_pinned(device: torch.device) -> bool:
+    """Whether an upload to ``device`` may go from pinned memory without waiting. Not into a
+    graph under capture: its replays would read the buffer after the caching host
+    allocator has given it to someone else; a pageable copy refuses the capture."""
+    return device.type == "cuda" and not torch.cuda.is_current_stream_capturing()
+
+
 def require_device(*tensors: torch.Tensor, what: str = "fused selected-quant decode") -> torch.device:
     """All tensors on one ROCm device, or RuntimeError (no host path exists)."""
     devs = {t.device for t in tensors if isinstance(t, torch.Tensor)}

@@ -29,7 +29,7 @@ import torch
 
 from . import _native as N
 from .block_router import RoutedBlock, _SELECTING
-from .decode_core import current_stream_handle
+from .decode_core import current_stream_handle, uploads_pinned
 from .fused_selected_quant_decode import FusedDecodeConfig, FusedKVPrecision, precision_tag
 from .intent_quant import KVPrecision
 
@@ -77,11 +77,12 @@ def _upload(arrays, dev: torch.device) -> List[torch.Tensor]:
         out.append(None)
         total += max(a.size, 1)              # a valid pointer for an empty array
     if host:
-        staged = torch.empty(total, dtype=torch.int32, pin_memory=True)
+        pinned = uploads_pinned(dev)
+        staged = torch.empty(total, dtype=torch.int32, pin_memory=pinned)
         view = staged.numpy()
         for _, at, a in host:
             view[at:at + max(a.size, 1)] = a if a.size else 0
-        sent = staged.to(dev, non_blocking=True)
+        sent = staged.to(dev, non_blocking=pinned)
         for i, at, a in host:
             out[i] = sent[at:at + max(a.size, 1)]
     return out

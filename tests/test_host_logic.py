@@ -269,3 +269,14 @@ def test_precision_enums_are_singletons_under_identity_hash():
             assert pickle.loads(pickle.dumps(m)) is m and copy.deepcopy(m) is m
             assert str(m) == m.value and len({m, enum(m.value)}) == 1
     assert ia.QuantPolicy(ia.KVPrecision.INT4_RESIDUAL).estimated_bytes_per_value == 1.0
+
+
+def test_uploads_are_not_pinned_into_a_capture(monkeypatch):
+    """A captured copy from pinned memory would replay from a buffer given back; the
+    pageable copy refuses the capture."""
+    import torch
+    from intent_attention import decode_core
+    for capturing in (False, True):
+        monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda c=capturing: c)
+        assert decode_core.uploads_pinned(torch.device("cuda", 0)) is not capturing
+        assert not decode_core.uploads_pinned(torch.device("cpu"))
