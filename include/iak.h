@@ -46,6 +46,8 @@
  *   iak_dense_attention         dense_attention() reference.py:16-45 (causal, mask, original_kv_positions),
  *                               under semantic_block_attention() reference.py:81-129 and
  *                               intent_quant_attention_reference() intent_quant_attention.py:20-119
+ *   iak_dense_attention_indexed the index_select of the selected tokens and that call, in
+ *                               semantic_block_attention() reference.py:100-112
  *   iak_dense_attention_workspace (no counterpart: sizes the optional split-over-keys and tile-flag buffer)
  *   iak_fake_quant_blocks       the per-block fake_quantize_tensor() reconstructions and their torch.cat
  *                               in intent_quant_attention_reference() intent_quant_attention.py:56-84
@@ -548,6 +550,12 @@ iak_status iak_dense_attention_workspace(const iak_dense_attention_args* args, s
 
 iak_status iak_dense_attention(const iak_dense_attention_args* args, void* workspace, size_t workspace_bytes,
                                void* stream);
+
+/* The same over selected tokens, read where they are: key j is row kv_index[j] of k and v
+ * (kv_index [kv_len] int64 on the device, or NULL: row j). The caller keeps every index
+ * non-negative, inside k and v and below 2^31; masks and positions stay by j. */
+iak_status iak_dense_attention_indexed(const iak_dense_attention_args* args, const int64_t* kv_index,
+                                       void* workspace, size_t workspace_bytes, void* stream);
 
 /* Fake-quant reconstruction of the selected blocks of float32 K and V, as
  * intent_quant_attention_reference() concatenates them (intent_quant_attention.py:56-84,

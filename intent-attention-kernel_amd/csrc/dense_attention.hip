@@ -18,6 +18,11 @@
 // 10.8 ms -> 0.10 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 18 us);
 // what follows is the rows form, for the rest.
 //
+// Selected tokens (kv_index) are read where they lie: the gathered K and V of 3,072 of
+// 4,096 tokens x 8 heads x 64 in float32 took two launches of 9 us and a pass over both,
+// the index in the kernel costs nothing that shows (blocks through
+// semantic_block_attention 170 -> 50 us with the index uploaded without a wait).
+//
 // Work split. A (batch, query) row's keys go to `splits` workgroups of
 // consecutive key ranges (`chunk` keys each); splits > 1 only when the caller
 // gives a workspace and there are few rows with 256 keys or more (decode shapes),
@@ -83,10 +88,15 @@ __device__ __forceinline__ void store_t(void* p, int64_t i, float x) {
   }
 }
 
+// the entry point's arguments, and the rows of k and v that are its keys (or null: key j is row j)
+struct DenseArgs : iak_dense_attention_args {
+  const int64_t* kv_index;
+};
+
 // the mask values of keys j0 .. j0 + KEYS - 1 of one query row (indices
 // clamped to the range's last key `last`)
 template <typename M, int KEYS>
-__device__ __forceinline__ void step_mask(const iak_dense_attention_args& a, int64_t mb, int j0, int last,
+__device__ __forceinline__ void step_mask(const DenseArgs& a, int64_t mb, int j0, int last,
                                           float* madd) {
 #pragma unroll
   for (int u = 0; u < KEYS; ++u) {
@@ -125,7 +135,7 @@ struct DenseSplit {
 // are at most 64 * NPL); KEYS keys per wave and step; WAVES waves per workgroup.
 // `item` = row * splits + split, row = b * q_len + i; `items` of them in all.
 template <typename T, int NPL, int KEYS, int WAVES>
-__device__ __forceinline__ void dense_row(const iak_dense_attention_args& a, const DenseSplit& sp, int64_t item,
+__device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& sp, int64_t item,
                                           int64_t items) {
   __shared__ float part_acc[WAVES][64 * NPL];
   __shared__ float part_m[WAVES], part_l[WAVES];
@@ -168,8 +178,9 @@ __device__ __forceinline__ void dense_row(const iak_dense_attention_args& a, con
 #pragma unroll
     for (int u = 0; u < KEYS; ++u) {
       const int jc = j0 + u < hi ? j0 + u : hi - 1;
-      const T* kr = kbase + (int64_t)jc * a.k_stride_t;
-      const T* vr = vbase + (int64_t)jc * a.v_stride_t;
+      const int64_t at = a.kv_index ? a.kv_index[jc] : jc;   // wave-uniform
+      const T* kr = kbase + at * a.k_stride_t;
+      const T* vr = vbase + at * a.v_stride_t;
 #pragma unroll
       for (int jj = 0; jj < NPL; ++jj) {
         kn[u][jj] = to_f32(kr[dk[jj]]);
@@ -296,7 +307,7 @@ __device__ __forceinline__ void dense_row(const iak_dense_attention_args& a, con
 }
 
 template <typename T, int NPL, int KEYS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const iak_dense_attention_args a,
+__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const DenseArgs a,
                                                                       const DenseSplit sp) {
   dense_row<T, NPL, KEYS, WAVES>(a, sp, blockIdx.x, gridDim.x);
 }
@@ -330,7 +341,7 @@ __device__ __forceinline__ float block_reduce(float v, float* red) {
 // FLAGS: the partials come from dense_matrix_kernel with key-tile flags; a row of
 // a flagged batch entry is computed again from its inputs.
 template <typename T, bool FLAGS>
-__global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const iak_dense_attention_args a,
+__global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseArgs a,
                                                                     const DenseSplit sp, const MatrixPlan mp) {
   __shared__ float wt[MAX_SPLITS];
   __shared__ float red[MERGE_THREADS / 64];
@@ -398,7 +409,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const iak_de
 // MAXW: the most waves per workgroup whose registers and LDS fit (16 waves of
 // a 1,024-thread workgroup get 128 VGPRs each)
 template <typename T, int NPL, int KEYS, int MAXW>
-void launch_items(const iak_dense_attention_args& a, const DenseSplit& sp, int64_t items, hipStream_t stream) {
+void launch_items(const DenseArgs& a, const DenseSplit& sp, int64_t items, hipStream_t stream) {
   // waves per workgroup: about 4,096 waves in the grid (16 per CU), between 4 and MAXW
   const int64_t want = (4096 + items - 1) / items;
   const dim3 grid((unsigned)items);
@@ -412,7 +423,7 @@ void launch_items(const iak_dense_attention_args& a, const DenseSplit& sp, int64
 }
 
 template <typename T>
-void launch_rows(const iak_dense_attention_args& a, const DenseSplit& sp, hipStream_t stream) {
+void launch_rows(const DenseArgs& a, const DenseSplit& sp, hipStream_t stream) {
   const int64_t rows = (int64_t)a.batch * a.q_len;
   const int64_t items = rows * sp.splits;
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
@@ -432,7 +443,7 @@ void launch_rows(const iak_dense_attention_args& a, const DenseSplit& sp, hipStr
 // than 512 rows) go over about SPLIT_TARGET_WGS workgroups in ranges of at
 // least RANGE_MIN_KEYS keys
 // (at most MAX_SPLITS ranges).
-DenseSplit split_plan(const iak_dense_attention_args& a) {
+DenseSplit split_plan(const DenseArgs& a) {
   DenseSplit sp{1, a.kv_len, nullptr, 0, 0};
   const int64_t rows = (int64_t)a.batch * a.q_len;
   if (rows <= 0 || rows >= 512 || a.kv_len < SPLIT_MIN_KEYS) return sp;
@@ -471,7 +482,7 @@ struct MatrixShape {
 };
 
 // 16-byte pieces of whole elements on every operand, at most 256 dims
-bool matrix_applies(const iak_dense_attention_args& a) {
+bool matrix_applies(const DenseArgs& a) {
   const int es = a.dtype == IAK_DTYPE_F32 ? 4 : 2, vec = 16 / es;
   const double pairs = (double)a.batch * a.q_len * a.kv_len;
   if (a.q_len < (es == 4 ? MX_MIN_ROWS_F32 : MX_MIN_ROWS) || pairs < (es == 4 ? MX_MIN_PAIRS_F32 : MX_MIN_PAIRS)) return false;
@@ -488,7 +499,7 @@ bool matrix_applies(const iak_dense_attention_args& a) {
   return true;
 }
 
-MatrixShape matrix_shape(const iak_dense_attention_args& a) {
+MatrixShape matrix_shape(const DenseArgs& a) {
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
   MatrixShape s{64, 4, 1, 64};
   const bool f32 = a.dtype == IAK_DTYPE_F32;
@@ -502,7 +513,7 @@ MatrixShape matrix_shape(const iak_dense_attention_args& a) {
 
 // query tiles of 32 * qw rows; on short grids the keys go over about 256
 // workgroups in ranges of whole tiles
-MatrixPlan matrix_plan(const iak_dense_attention_args& a, const MatrixShape& s) {
+MatrixPlan matrix_plan(const DenseArgs& a, const MatrixShape& s) {
   MatrixPlan mp{};
   const int64_t bq = 32 * s.qw, bk = s.kw * s.bkw;
   mp.nq = (int)((a.q_len + bq - 1) / bq);
@@ -520,16 +531,16 @@ MatrixPlan matrix_plan(const iak_dense_attention_args& a, const MatrixShape& s) 
 }
 
 // key-tile flags are needed where a weight is split or tiles are skipped
-bool matrix_flags(const iak_dense_attention_args& a, const MatrixPlan& mp) {
+bool matrix_flags(const DenseArgs& a, const MatrixPlan& mp) {
   return a.dtype != IAK_DTYPE_F32 || mp.skip;
 }
 
-size_t matrix_partial_bytes(const iak_dense_attention_args& a, const MatrixPlan& mp) {
+size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
   if (mp.splits <= 1) return 0;
   return ((size_t)mp.accoff + (size_t)a.batch * a.q_len * mp.splits * (size_t)a.v_dim) * sizeof(float);
 }
 
-size_t matrix_workspace(const iak_dense_attention_args& a) {
+size_t matrix_workspace(const DenseArgs& a) {
   const MatrixPlan mp = matrix_plan(a, matrix_shape(a));
   const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * 4 * sizeof(int32_t) : 0;
   const size_t total = matrix_partial_bytes(a, mp) + flags;
@@ -537,7 +548,7 @@ size_t matrix_workspace(const iak_dense_attention_args& a) {
 }
 
 template <typename T, int DP, int QW, int KW, int BKW>
-void launch_matrix_cfg(const iak_dense_attention_args& a, const MatrixPlan& mp, hipStream_t stream) {
+void launch_matrix_cfg(const DenseArgs& a, const MatrixPlan& mp, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)a.batch * mp.nq * mp.splits));
   if (a.mask || a.causal == IAK_CAUSAL_POSITIONS)
     hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, true>), grid, dim3(MX_THREADS), 0, stream,
@@ -548,7 +559,7 @@ void launch_matrix_cfg(const iak_dense_attention_args& a, const MatrixPlan& mp, 
 }
 
 template <typename T, int DP>
-void launch_matrix_dims(const iak_dense_attention_args& a, const MatrixShape& s, const MatrixPlan& mp,
+void launch_matrix_dims(const DenseArgs& a, const MatrixShape& s, const MatrixPlan& mp,
                         hipStream_t stream) {
   constexpr int BKW = sizeof(T) == 4 ? 32 : 64;
   if constexpr (DP <= 128) {
@@ -559,7 +570,7 @@ void launch_matrix_dims(const iak_dense_attention_args& a, const MatrixShape& s,
 }
 
 template <typename T>
-void launch_matrix(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
+void launch_matrix(const DenseArgs& a, void* workspace, hipStream_t stream) {
   const MatrixShape s = matrix_shape(a);
   MatrixPlan mp = matrix_plan(a, s);
   mp.ws = static_cast<float*>(workspace);
@@ -587,7 +598,7 @@ void launch_matrix(const iak_dense_attention_args& a, void* workspace, hipStream
 }
 
 template <typename T>
-void launch_typed(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
+void launch_typed(const DenseArgs& a, void* workspace, hipStream_t stream) {
   if (workspace && matrix_applies(a)) return launch_matrix<T>(a, workspace, stream);
   DenseSplit sp = split_plan(a);
   if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr, 0, 0};
@@ -597,14 +608,17 @@ void launch_typed(const iak_dense_attention_args& a, void* workspace, hipStream_
 
 }  // namespace
 
-size_t dense_attention_workspace(const iak_dense_attention_args& a) {
+size_t dense_attention_workspace(const iak_dense_attention_args& args) {
+  const DenseArgs a{args, nullptr};   // the keys' rows change no size
   const DenseSplit sp = split_plan(a);
   const size_t rows = sp.splits <= 1 ? 0 : (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.v_dim) * sizeof(float);
   const size_t matrix = matrix_applies(a) ? matrix_workspace(a) : 0;
   return rows > matrix ? rows : matrix;
 }
 
-hipError_t launch_dense_attention(const iak_dense_attention_args& a, void* workspace, hipStream_t stream) {
+hipError_t launch_dense_attention(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
+                                  hipStream_t stream) {
+  const DenseArgs a{args, kv_index};
   if (a.dtype == IAK_DTYPE_F32) launch_typed<float>(a, workspace, stream);
   else if (a.dtype == IAK_DTYPE_F16) launch_typed<_Float16>(a, workspace, stream);
   else launch_typed<bf16_bits>(a, workspace, stream);

@@ -197,7 +197,7 @@ template <typename T, int DP, int QW, int KW, int BKW, bool GEN> struct MxCfg {
 
 template <typename T, int DP, int QW, int KW, int BKW, bool GEN>
 __global__ __launch_bounds__(MX_THREADS, (sizeof(T) == 2 ? DP <= 128 && KW == 1 : DP <= 64) ? 2 : 1)
-void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) {
+void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
   using C = MxCfg<T, DP, QW, KW, BKW, GEN>;
   using E = MxElem<T>;
   using vec = typename E::vec;
@@ -273,20 +273,30 @@ void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) 
     c = f - r * CH;
     if (C::PRIV) r += kw * BKW;
   };
-  // the tile's pieces (rows past the range repeat its last key, dims past the
-  // width are zero)
-  auto load_pieces = [&](u4* x, const T* base, int64_t stride, int width, int t) {
+  // K and V rows of the pieces of tile t (rows past the range repeat its last key),
+  // looked up one tile ahead where the keys are an index
+  int at[NCH];
+  auto look_up = [&](int t) {
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
       int r, c;
       piece(i, r, c);
       const int j0 = lo + t * BK + r, j = j0 < hi ? j0 : hi - 1;
-      x[i] = u4{0u, 0u, 0u, 0u};
-      if (c * C::EPC < width) x[i] = *reinterpret_cast<const u4*>(base + (int64_t)j * stride + c * C::EPC);
+      at[i] = a.kv_index ? (int)a.kv_index[j] : j;
     }
   };
-  auto load_k = [&](int t) { load_pieces(kr, kbase, a.k_stride_t, a.head_dim, t); };
-  auto load_v = [&](int t) { load_pieces(C::STAGED ? kr : vr, vbase, a.v_stride_t, a.v_dim, t); };
+  // the pieces of the tile looked up last (dims past the width are zero)
+  auto load_pieces = [&](u4* x, const T* base, int64_t stride, int width) {
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      int r, c;
+      piece(i, r, c);
+      x[i] = u4{0u, 0u, 0u, 0u};
+      if (c * C::EPC < width) x[i] = *reinterpret_cast<const u4*>(base + (int64_t)at[i] * stride + c * C::EPC);
+    }
+  };
+  auto load_k = [&]() { load_pieces(kr, kbase, a.k_stride_t, a.head_dim); };
+  auto load_v = [&]() { load_pieces(C::STAGED ? kr : vr, vbase, a.v_stride_t, a.v_dim); };
   auto large = [&](const u4* x) {
     bool bad = false;
 #pragma unroll
@@ -511,23 +521,26 @@ void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) 
   if constexpr (C::STAGED) {
     bool bad = false;
     if (tiles > 0) {
-      load_k(0);
+      look_up(0);
+      load_k();
       if (mp.flags) bad = large(kr);
       store_k(0);
-      load_v(0);
+      load_v();
+      if (tiles > 1) look_up(1);
       if (checks(0)) put_flag(0, bad || large(kr));
       store_v(0);
     }
     for (int t = 0; t < tiles; ++t) {
       const bool more = t + 1 < tiles;
       sync();   // tile t is in place
-      if (more) load_k(t + 1);
+      if (more) load_k();
       if (seen(t)) scores(t, 0);
       sync();   // its keys are read
       if (more) {
         if (mp.flags) bad = large(kr);
         store_k(0);
-        load_v(t + 1);
+        load_v();
+        if (t + 2 < tiles) look_up(t + 2);
       }
       if (seen(t)) values(t, 0);
       sync();   // its values are read
@@ -538,8 +551,10 @@ void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) 
     }
   } else {
     if (tiles > 0) {
-      load_k(0);
-      load_v(0);
+      look_up(0);
+      load_k();
+      load_v();
+      if (tiles > 1) look_up(1);
       if (checks(0)) put_flag(0, large(kr) || large(vr));
       store_k(0);
       store_v(0);
@@ -549,8 +564,9 @@ void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) 
       const int buf = C::NB == 2 ? t & 1 : 0, next = C::NB == 2 ? buf ^ 1 : 0;
       sync();   // tile t is in place; with two buffers, the other one is free
       if (more) {
-        load_k(t + 1);
-        load_v(t + 1);
+        load_k();
+        load_v();
+        if (t + 2 < tiles) look_up(t + 2);
       }
       if (seen(t)) {
         scores(t, buf);
@@ -570,9 +586,10 @@ void dense_matrix_kernel(const iak_dense_attention_args a, const MatrixPlan mp) 
     for (int t = 0; t < all; ++t) {
       const int64_t g = lo / BK + t;
       if (g * BK / C::BQ >= mp.nq && g % mp.nq == qt) {
-        load_k(t);
+        look_up(t);
+        load_k();
         bool bad = large(kr);
-        load_v(t);
+        load_v();
         if constexpr (C::STAGED) bad |= large(kr);
         else bad |= large(vr);
         put_flag(t, bad);
@@ -677,7 +694,7 @@ __device__ __forceinline__ bool mx_flagged(const MatrixPlan& mp, int64_t b) {
 // Workgroup g: batch entry g % batch, every (grid / batch)-th of its rows, and
 // only if one of its key tiles is flagged.
 template <typename T>
-__global__ __launch_bounds__(256) void dense_fixup_kernel(const iak_dense_attention_args a, const MatrixPlan mp) {
+__global__ __launch_bounds__(256) void dense_fixup_kernel(const DenseArgs a, const MatrixPlan mp) {
   const int64_t b = blockIdx.x % (unsigned)a.batch, first = blockIdx.x / (unsigned)a.batch;
   if (!mx_flagged(mp, b)) return;
   const DenseSplit one{1, a.kv_len, nullptr, 0, 0};

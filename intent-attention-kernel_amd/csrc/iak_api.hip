@@ -374,7 +374,7 @@ size_t mla_rows_workspace(const iak_mla_rows_args& a);                          
 hipError_t launch_fake_quant_blocks(const iak_fake_quant_blocks_args& a, void* workspace,
                                     hipStream_t stream);                    // fake_quant.hip
 size_t fake_quant_blocks_workspace(const iak_fake_quant_blocks_args& a);   // fake_quant.hip
-hipError_t launch_dense_attention(const iak_dense_attention_args& a, void* workspace,
+hipError_t launch_dense_attention(const iak_dense_attention_args& a, const int64_t* kv_index, void* workspace,
                                   hipStream_t stream);                     // dense_attention.hip
 size_t dense_attention_workspace(const iak_dense_attention_args& a);     // dense_attention.hip
 }
@@ -831,6 +831,11 @@ iak_status iak_dense_attention_workspace(const iak_dense_attention_args* a, size
 
 iak_status iak_dense_attention(const iak_dense_attention_args* a, void* workspace, size_t workspace_bytes,
                                void* stream) {
+  return iak_dense_attention_indexed(a, nullptr, workspace, workspace_bytes, stream);
+}
+
+iak_status iak_dense_attention_indexed(const iak_dense_attention_args* a, const int64_t* kv_index, void* workspace,
+                                       size_t workspace_bytes, void* stream) {
   const iak_status st = validate_dense(a);
   if (st != IAK_OK) return st;
   if ((long long)a->batch * a->q_len == 0) return IAK_OK;
@@ -840,7 +845,7 @@ iak_status iak_dense_attention(const iak_dense_attention_args* a, void* workspac
       return fail(IAK_EINVAL, "workspace of %zu bytes is smaller than the %zu bytes required", workspace_bytes, need);
     if (!aligned16(workspace)) return fail(IAK_EINVAL, "workspace must be 16-byte aligned");
   }
-  const hipError_t e = iak::launch_dense_attention(*a, workspace, static_cast<hipStream_t>(stream));
+  const hipError_t e = iak::launch_dense_attention(*a, kv_index, workspace, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(IAK_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
   return IAK_OK;
 }

@@ -184,7 +184,7 @@ EXPORTED = ("iak_abi_version", "iak_status_string", "iak_last_error",
             "iak_build_page_tables", "iak_paged_decode_timed", "iak_mla_decode_timed",
             "iak_paged_decode_noalloc", "iak_transcode_pages", "iak_prefetch_pages", "iak_paged_decode_plan",
             "iak_mla_decode_rows", "iak_pack_page_descriptors",
-            "iak_pack_entry_records", "iak_dense_attention", "iak_dense_attention_workspace",
+            "iak_pack_entry_records", "iak_dense_attention", "iak_dense_attention_indexed", "iak_dense_attention_workspace",
             "iak_mla_decode_rows_workspace", "iak_fake_quant_blocks",
             "iak_fake_quant_blocks_workspace", "iak_timing_event_create", "iak_timing_event_record",
             "iak_timing_event_elapsed", "iak_timing_event_destroy")
@@ -263,6 +263,9 @@ def load() -> ctypes.CDLL:
     lib.iak_pack_page_descriptors.argtypes = [ctypes.POINTER(PagedDecodeArgs), c_void_p, c_void_p]
     lib.iak_dense_attention.restype = ctypes.c_int
     lib.iak_dense_attention.argtypes = [ctypes.POINTER(DenseAttentionArgs), c_void_p, ctypes.c_size_t, c_void_p]
+    lib.iak_dense_attention_indexed.restype = ctypes.c_int
+    lib.iak_dense_attention_indexed.argtypes = [ctypes.POINTER(DenseAttentionArgs), c_void_p, c_void_p,
+                                                ctypes.c_size_t, c_void_p]
     lib.iak_dense_attention_workspace.restype = ctypes.c_int
     lib.iak_dense_attention_workspace.argtypes = [ctypes.POINTER(DenseAttentionArgs), ctypes.POINTER(ctypes.c_size_t)]
     lib.iak_pack_entry_records.restype = ctypes.c_int
@@ -427,5 +430,7 @@ def dense_attention_workspace(args: DenseAttentionArgs) -> int:
     return int(n.value)
 
 
-def dense_attention(args: DenseAttentionArgs, stream: int, workspace: int = 0, workspace_bytes: int = 0) -> None:
-    check(load().iak_dense_attention(ctypes.byref(args), workspace or None, workspace_bytes, stream or None))
+def dense_attention(args: DenseAttentionArgs, stream: int, workspace: int = 0, workspace_bytes: int = 0,
+                    kv_index: int = 0) -> None:
+    check(load().iak_dense_attention_indexed(ctypes.byref(args), kv_index or None, workspace or None, workspace_bytes,
+                                             stream or None))

@@ -38,11 +38,12 @@ from __future__ import annotations
 import math
 from typing import Any, Dict, List, Optional, Tuple, Union
 
+import numpy as np
 import torch
 
 from . import _native as N
 from .block_metadata import BlockLayout, BlockPolicy
-from .decode_core import current_stream_handle, require_device
+from .decode_core import current_stream_handle, require_device, uploads_pinned
 
 _DTYPES = {torch.float16: N.DTYPE_F16, torch.float32: N.DTYPE_F32, torch.bfloat16: N.DTYPE_BF16}
 _MAX_DIM = 1024
@@ -68,6 +69,13 @@ def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
                     mask: Optional[torch.Tensor] = None,
                     original_kv_positions: Optional[torch.Tensor] = None) -> torch.Tensor:
     """softmax(q k^T / sqrt(D) [+ causal mask] [+ mask]) v over [..., T, D] tensors, on the HIP kernel."""
+    return _dense_attention(q, k, v, causal, mask, original_kv_positions)
+
+
+def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: bool, mask: Optional[torch.Tensor],
+                     original_kv_positions: Optional[torch.Tensor],
+                     kv_index: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``dense_attention``; with ``kv_index`` (int64, inside k and v) over those rows of k and v."""
     dev = require_device(*(t for t in (q, k, v, mask, original_kv_positions) if t is not None),
                          what="dense attention")
     if q.dim() < 2 or k.dim() < 2 or v.dim() < 2:
@@ -76,10 +84,10 @@ def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
         raise RuntimeError(f"expected m1 and m2 to have the same dtype, but got: {_dtype_name(q.dtype)} != "
                            f"{_dtype_name(k.dtype)}")
     D, Dv = q.shape[-1], v.shape[-1]
-    Tq, Tk = q.shape[-2], k.shape[-2]
+    Tq, Tk = q.shape[-2], k.shape[-2] if kv_index is None else kv_index.shape[0]
     if k.shape[-1] != D:
         raise RuntimeError(f"q and k head dims differ: {D} != {k.shape[-1]}")
-    if v.shape[-2] != Tk:
+    if kv_index is None and v.shape[-2] != Tk:
         raise RuntimeError(f"k and v lengths differ: {Tk} != {v.shape[-2]}")
     score_dtype = q.dtype if mask is None else torch.promote_types(q.dtype, mask.dtype)
     if score_dtype != v.dtype:
@@ -139,7 +147,8 @@ def dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: b
     # allocator reuses their memory only after these kernels
     ws_bytes = N.dense_attention_workspace(a)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
-    N.dense_attention(a, current_stream_handle(dev), ws.data_ptr() if ws is not None else 0, ws_bytes)
+    N.dense_attention(a, current_stream_handle(dev), ws.data_ptr() if ws is not None else 0, ws_bytes,
+                      kv_index.data_ptr() if kv_index is not None else 0)
     return out
 
 
@@ -163,6 +172,22 @@ def _resolve_dynamic_scores(q: torch.Tensor, k: torch.Tensor, layout: BlockLayou
     return dynamic
 
 
+def _token_index(spans: List[Tuple[int, int]], dev: torch.device) -> torch.Tensor:
+    """The token indices of the spans in order, int64 on the device."""
+    idx = torch.from_numpy(np.concatenate([np.arange(s, e, dtype=np.int64) for s, e in spans]))
+    if not uploads_pinned(dev):
+        return idx.to(dev)
+    return idx.pin_memory().to(dev, non_blocking=True)
+
+
+def _index_in_place(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
+    """Whether the kernel can read the selected rows of k and v where they are: equal
+    leading shapes and contiguous, aligned rows (an index_select makes them so)."""
+    return (k.dim() >= 2 and q.shape[:-2] == k.shape[:-2] == v.shape[:-2] and v.shape[-2] == k.shape[-2]
+            and k.shape[-2] < 2 ** 31 and k.is_contiguous() and v.is_contiguous()
+            and k.data_ptr() % 16 == 0 and v.data_ptr() % 16 == 0)
+
+
 def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layout: BlockLayout,
                              causal: bool = False, return_debug: bool = False,
                              threshold: float = 0.5) -> Union[torch.Tensor, Tuple[torch.Tensor, Dict[str, Any]]]:
@@ -172,8 +197,8 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     kv_tokens = k.size(-2)
     dynamic = _resolve_dynamic_scores(q, k, layout)
     layout.validate(kv_tokens)
-    selected: List[int] = layout.selected_token_indices()
-    if not selected:
+    spans = [(b.start, b.end) for b in layout.selected_blocks()]
+    if not spans:
         out = torch.zeros_like(q)
         if not return_debug:
             return out
@@ -182,14 +207,17 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         if dynamic:
             debug["dynamic_scores"] = dynamic
         return out, debug
-    idx = torch.tensor(selected, dtype=torch.long, device=k.device)
-    out = dense_attention(q, k.index_select(-2, idx), v.index_select(-2, idx), causal=causal,
-                          original_kv_positions=idx)
+    idx = _token_index(spans, k.device)
+    if _index_in_place(q, k, v):
+        out = _dense_attention(q, k, v, causal, None, idx, kv_index=idx)
+    else:
+        out = dense_attention(q, k.index_select(-2, idx), v.index_select(-2, idx), causal=causal,
+                              original_kv_positions=idx)
     if not return_debug:
         return out
     debug = {"selected_token_count": layout.selected_token_count(),
              "selected_block_names": [b.name for b in layout.selected_blocks()],
-             "total_kv_tokens": kv_tokens, "selected_kv_tokens": len(selected)}
+             "total_kv_tokens": kv_tokens, "selected_kv_tokens": int(idx.shape[0])}
     if dynamic:
         debug["dynamic_scores"] = dynamic
     return out, debug

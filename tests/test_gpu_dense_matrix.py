@@ -127,3 +127,33 @@ def test_replays_from_a_graph():
         want = dense_attention(qc, kc, vc, causal=True)
         torch.cuda.synchronize()
         assert torch.equal(out, want) and not torch.equal(out, eager), i
+
+
+# rows form (1 row, few pairs), split rows, and the three wave shapes of the matrix form; head
+# dims with and without 16-byte rows
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("tq,d", [(1, 64), (3, 20), (5, 128), (40, 64), (128, 64), (130, 96)])
+def test_selected_blocks_read_in_place(tq, d, dt):
+    """Keys read through the selected tokens' index are bit for bit the gathered keys' result,
+    NaN and infinity in and outside the selection included."""
+    from intent_attention import BlockLayout, BlockPolicy, SemanticBlock, dense_attention, semantic_block_attention
+    spans = [(0, 3), (5, 64), (64, 65), (130, 700), (901, 1000)]
+    layout = BlockLayout([SemanticBlock(f"b{i}", s, e, BlockPolicy.ALWAYS) for i, (s, e) in enumerate(spans)])
+    sel = torch.tensor([t for s, e in spans for t in range(s, e)]).cuda()
+    lead = (2, 8)
+    q, k, v, _ = (x.cuda() if isinstance(x, torch.Tensor) else x for x in _qkv(tq + d, lead, tq, 1000, d, d, dt))
+    k[:, :, 800] = float("nan")             # not selected
+    v[:, :, 4] = float("inf")
+    for case in ("finite", "inf in v", "strided"):
+        if case == "inf in v":
+            v[1, 3, 699] = float("inf")
+        if case == "strided":               # not read in place
+            k = k.transpose(0, 1).contiguous().transpose(0, 1)
+        for causal in (False, True):
+            want = dense_attention(q, k.index_select(-2, sel), v.index_select(-2, sel), causal=causal,
+                                   original_kv_positions=sel)
+            got, debug = semantic_block_attention(q, k, v, layout, causal=causal, return_debug=True)
+            assert torch.equal(torch.nan_to_num(got, 7.0, 8.0, -8.0), torch.nan_to_num(want, 7.0, 8.0, -8.0)), case
+            assert debug["selected_kv_tokens"] == debug["selected_token_count"] == sel.numel()
+            if case == "finite" and not causal:
+                assert bool(got.isfinite().all())
