@@ -15,7 +15,7 @@
 //
 // Calls with several query rows per batch entry run on the matrix cores
 // (dense_matrix.h: causal prefill of 32 heads x 2,048 rows x 128 in float16
-// 10.8 ms -> 0.10 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 18 us);
+// 10.8 ms -> 0.082 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 18 us);
 // what follows is the rows form, for the rest.
 //
 // Selected tokens (kv_index) are read where they lie: the gathered K and V of 3,072 of
@@ -475,6 +475,19 @@ DenseSplit split_plan(const DenseArgs& a) {
 #define MX_MIN_ROWS_F32 3
 #endif
 
+// 128 query rows by four waves over 64 keys, or by eight over 128: a step of one wave per
+// SIMD takes 3 us, of two (two workgroups on a CU, or the eight waves of one) 2.2 us for
+// each 64 keys, the one's matrix work under the other's softmax. Up to one workgroup per
+// CU the eight waves are the only way to two (float16, 16 heads x 2,048 x 128: 100 ->
+// 72 us; 32 heads, two workgroups per CU: 138 / 144). A causal grid is bound by its
+// longest tiles, which run alone when the short ones have ended; eight waves halve them
+// (32 heads x 2,048 x 128: 98 -> 82 us, 3 x 4,096 x 128: 135 -> 100, 32 x 4,096 x
+// 128, 1,024 workgroups: 282 / 297).
+#ifndef MX_WIDE_WGS
+#define MX_WIDE_WGS 256
+#define MX_WIDE_WGS_CAUSAL 512
+#endif
+
 struct MatrixShape {
   int dp;       // dims, padded
   int qw, kw;   // waves over query rows and over keys
@@ -499,6 +512,9 @@ bool matrix_applies(const DenseArgs& a) {
   return true;
 }
 
+// causal tiles past the diagonal are not visited
+bool causal_skip(const DenseArgs& a) { return a.causal == IAK_CAUSAL_TRIU && !a.mask && a.sm_scale <= 1.f; }
+
 MatrixShape matrix_shape(const DenseArgs& a) {
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
   MatrixShape s{64, 4, 1, 64};
@@ -508,6 +524,8 @@ MatrixShape matrix_shape(const DenseArgs& a) {
   // few query rows: the four waves share out the keys instead
   if (a.q_len <= 32 && s.dp <= 128) s.qw = 1, s.kw = 4, s.bkw = 32;
   else if (a.q_len <= 64 && s.dp <= 128) s.qw = 2, s.kw = 2, s.bkw = 32;
+  else if (!f32 && s.dp <= 128 && a.kv_len > 128 &&
+           (int64_t)a.batch * ((a.q_len + 127) / 128) <= (causal_skip(a) ? MX_WIDE_WGS_CAUSAL : MX_WIDE_WGS)) s.kw = 2;
   return s;
 }
 
@@ -518,7 +536,8 @@ MatrixPlan matrix_plan(const DenseArgs& a, const MatrixShape& s) {
   const int64_t bq = 32 * s.qw, bk = s.kw * s.bkw;
   mp.nq = (int)((a.q_len + bq - 1) / bq);
   mp.nt = (int)((a.kv_len + bk - 1) / bk);
-  mp.skip = a.causal == IAK_CAUSAL_TRIU && !a.mask && a.sm_scale <= 1.f;
+  mp.waves = s.qw * s.kw;
+  mp.skip = causal_skip(a);
   const int64_t wgs = (int64_t)a.batch * mp.nq;
   int64_t n = wgs > 0 && wgs < SPLIT_TARGET_WGS ? SPLIT_TARGET_WGS / wgs : 1;
   if (n > mp.nt) n = mp.nt;
@@ -542,7 +561,7 @@ size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
 
 size_t matrix_workspace(const DenseArgs& a) {
   const MatrixPlan mp = matrix_plan(a, matrix_shape(a));
-  const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * 4 * sizeof(int32_t) : 0;
+  const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * mp.waves * sizeof(int32_t) : 0;
   const size_t total = matrix_partial_bytes(a, mp) + flags;
   return total ? total : 16;   // a workspace at all says that the form may run
 }
@@ -551,10 +570,10 @@ template <typename T, int DP, int QW, int KW, int BKW>
 void launch_matrix_cfg(const DenseArgs& a, const MatrixPlan& mp, hipStream_t stream) {
   const dim3 grid((unsigned)((int64_t)a.batch * mp.nq * mp.splits));
   if (a.mask || a.causal == IAK_CAUSAL_POSITIONS)
-    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, true>), grid, dim3(MX_THREADS), 0, stream,
+    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, true>), grid, dim3(64 * QW * KW), 0, stream,
                        a, mp);
   else
-    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, false>), grid, dim3(MX_THREADS), 0, stream,
+    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, false>), grid, dim3(64 * QW * KW), 0, stream,
                        a, mp);
 }
 
@@ -563,6 +582,9 @@ void launch_matrix_dims(const DenseArgs& a, const MatrixShape& s, const MatrixPl
                         hipStream_t stream) {
   constexpr int BKW = sizeof(T) == 4 ? 32 : 64;
   if constexpr (DP <= 128) {
+    if constexpr (sizeof(T) == 2) {
+      if (s.qw == 4 && s.kw == 2) return launch_matrix_cfg<T, DP, 4, 2, 64>(a, mp, stream);
+    }
     if (s.kw == 4) return launch_matrix_cfg<T, DP, 1, 4, 32>(a, mp, stream);
     if (s.kw == 2) return launch_matrix_cfg<T, DP, 2, 2, 32>(a, mp, stream);
   }

@@ -1,10 +1,11 @@
 // Tiled dense attention on the matrix cores: the form of dense_attention.hip
 // for several query rows per batch entry. Included by that file only.
 //
-// A workgroup of four waves takes QW x 32 query rows of one batch entry and
-// walks key tiles of KW x BKW keys; wave (qw, kw) owns 32 query rows and the
-// kw-th BKW keys of every tile (KW > 1 keeps all four waves busy when there
-// are few query rows; the waves' partial results meet in the LDS at the end).
+// A workgroup of QW x KW (four or eight) waves takes QW x 32 query rows of one
+// batch entry and walks key tiles of KW x BKW keys; wave (qw, kw) owns 32 query
+// rows and the kw-th BKW keys of every tile (KW > 1 keeps the waves busy when
+// there are few query rows, and puts two on a SIMD when there are few workgroups;
+// the waves' partial results meet in the LDS at the end).
 // K and V tiles go through registers into the LDS as they lie in memory, the
 // next tile's loads in flight while this tile is computed.
 //   scores  S^T[32 keys x 32 rows] = K . Q^T: A operand K[key = lane % 32], B
@@ -37,7 +38,6 @@
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
-constexpr int MX_THREADS = 256;
 constexpr int MX_MAX_DIM = 256;      // 16-bit inputs
 constexpr int MX_MAX_DIM_F32 = 128;  // float32: Q, scores and context of wider rows spill
 constexpr float LOG2E = 1.44269504088896340736f;
@@ -54,7 +54,8 @@ struct MatrixPlan {
   int skip;        // causal: tiles past the diagonal are not visited
   int64_t accoff;  // offset of the partial contexts in ws (floats)
   float* ws;       // splits > 1: the partials
-  int32_t* flags;  // [batch][nt][4 waves], or null (nothing to check)
+  int waves;       // waves of a workgroup
+  int32_t* flags;  // [batch][nt][waves], or null (nothing to check)
 };
 
 template <typename T> struct MxElem;   // operand vector of 16 bytes, matrix product, parts of a weight
@@ -172,7 +173,8 @@ __device__ __forceinline__ f16v mx_score_tree(const char* kt, int koff, const f4
 }
 
 template <typename T, int DP, int QW, int KW, int BKW, bool GEN> struct MxCfg {
-  static_assert(QW * KW == 4 && BKW % 32 == 0 && DP % 32 == 0, "four waves, whole 32 x 32 tiles");
+  static_assert((QW * KW == 4 || QW * KW == 8) && BKW % 32 == 0 && DP % 32 == 0, "whole 32 x 32 tiles");
+  static constexpr int THREADS = 64 * QW * KW;
   static constexpr int ES = sizeof(T);
   static constexpr int RB = DP * ES;               // LDS row bytes
   static constexpr int CH = RB / 16;               // 16-byte pieces per row
@@ -189,14 +191,14 @@ template <typename T, int DP, int QW, int KW, int BKW, bool GEN> struct MxCfg {
   // so the waves need no barrier
   static constexpr bool PRIV = QW == 1;
   static constexpr int LDS = NB * 2 * TILE;
-  static constexpr int NCH = BK * CH / MX_THREADS; // pieces per thread and tile
+  static constexpr int NCH = BK * CH / THREADS; // pieces per thread and tile
   static constexpr int NSB = BKW / 32, NDV = DP / 32;
-  static_assert(BK * CH % MX_THREADS == 0, "whole pieces per thread");
+  static_assert(BK * CH % THREADS == 0, "whole pieces per thread");
   static_assert(KW == 1 || KW * 32 * QW * DP * 4 <= LDS, "the waves' contexts meet in the tile buffers");
 };
 
 template <typename T, int DP, int QW, int KW, int BKW, bool GEN>
-__global__ __launch_bounds__(MX_THREADS, (sizeof(T) == 2 ? DP <= 128 && KW == 1 : DP <= 64) ? 2 : 1)
+__global__ __launch_bounds__(64 * QW * KW, (sizeof(T) == 2 ? DP <= 128 && QW == 4 : DP <= 64) ? 2 : 1)
 void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
   using C = MxCfg<T, DP, QW, KW, BKW, GEN>;
   using E = MxElem<T>;
@@ -220,12 +222,12 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
     const unsigned per = n >> 3, rem = n & 7u, nq = (unsigned)mp.nq, groups = n / nq;
     unsigned bs;
     if (mp.skip && (groups & 7u) == 0) {
-      // causal: the XCD's groups side by side, the longest query tiles first; on a
-      // grid that is resident at once (two workgroups per CU) the second half
-      // runs from the shortest, so each CU's two workgroups are about as long
-      // together (32 heads x 2,048 rows x 128: 85 us, longest first throughout 106)
+      // causal: the XCD's groups side by side, the longest query tiles first (32 heads x
+      // 4,096 rows x 128: 278 us; one group after the other 349); on a grid of
+      // two four-wave workgroups per CU, resident at once, the second half from the
+      // shortest, so each CU's two are about as long together
       const unsigned gpx = groups >> 3, half = (nq + 1) / 2 * gpx;
-      qt = (int)(n <= 512 && slot >= half ? (slot - half) / gpx : nq - 1 - slot / gpx);
+      qt = (int)(QW * KW == 4 && n <= 512 && slot >= half ? (slot - half) / gpx : nq - 1 - slot / gpx);
       bs = xcd * gpx + slot % gpx;
     } else {
       const unsigned item = xcd * per + (xcd < rem ? xcd : rem) + slot;
@@ -268,7 +270,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
   u4 kr[NCH], vr[C::STAGED ? 1 : NCH];
   // piece i of the thread: row and position in the tile
   auto piece = [&](int i, int& r, int& c) {
-    const int f = (C::PRIV ? lane : tid) + (C::PRIV ? 64 : MX_THREADS) * i;
+    const int f = (C::PRIV ? lane : tid) + (C::PRIV ? 64 : C::THREADS) * i;
     r = f / CH;
     c = f - r * CH;
     if (C::PRIV) r += kw * BKW;
@@ -306,7 +308,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
   // the flag of tile t of this range, by the workgroup whose turn it is (checks)
   auto put_flag = [&](int t, bool bad) {
     const bool any = __builtin_amdgcn_ballot_w64(bad) != 0;
-    if (lane == 0) mp.flags[((int64_t)b * mp.nt + lo / BK + t) * 4 + w] = any ? 1 : 0;
+    if (lane == 0) mp.flags[((int64_t)b * mp.nt + lo / BK + t) * (QW * KW) + w] = any ? 1 : 0;
   };
   auto checks = [&](int t) {
     if (!mp.flags) return false;
@@ -650,7 +652,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine[(32 * d + 8 * (r >> 2) + 4 * h + (r & 3)) * 32 + l32] = acc[d][r];
     __syncthreads();
-    // thread: row tid % BQ, every (256 / BQ)-th group of four dims
+    // thread: row tid % BQ, every (THREADS / BQ)-th group of four dims
     const int rq = tid % C::BQ, g0 = tid / C::BQ;
     const int r = q0 + rq;
     if (r >= a.q_len) return;
@@ -670,7 +672,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
       mp.ws[items + it] = L;
     }
     const float inv = F32 ? L : 1.0f / L;
-    for (int g = g0; g < DP / 4; g += MX_THREADS / C::BQ) {
+    for (int g = g0; g < DP / 4; g += C::THREADS / C::BQ) {
       f4 v = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < KW; ++k) {
@@ -686,8 +688,8 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
 // whether any key tile of batch entry b is flagged (workgroup-uniform)
 __device__ __forceinline__ bool mx_flagged(const MatrixPlan& mp, int64_t b) {
   int any = 0;
-  const int32_t* f = mp.flags + b * mp.nt * 4;
-  for (int64_t i = threadIdx.x; i < (int64_t)mp.nt * 4; i += blockDim.x) any |= f[i];
+  const int32_t* f = mp.flags + b * mp.nt * mp.waves;
+  for (int64_t i = threadIdx.x; i < (int64_t)mp.nt * mp.waves; i += blockDim.x) any |= f[i];
   return __syncthreads_or(any) != 0;
 }
 

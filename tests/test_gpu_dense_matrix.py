@@ -157,3 +157,21 @@ def test_selected_blocks_read_in_place(tq, d, dt):
             assert debug["selected_kv_tokens"] == debug["selected_token_count"] == sel.numel()
             if case == "finite" and not causal:
                 assert bool(got.isfinite().all())
+
+
+# both sides of the eight-wave rule (256 workgroups; causal 512; more than 128 keys), with
+# ragged rows and keys; 8 query tiles x 65 heads is one group per XCD and a remainder
+@pytest.mark.parametrize("dt", ["f16", "bf16"])
+@pytest.mark.parametrize("heads,t,tk,d", [(64, 512, 512, 64), (129, 130, 257, 96), (128, 129, 129, 128),
+                                          (257, 66, 300, 64), (65, 1000, 1000, 64), (3, 700, 128, 128)])
+def test_waves_per_workgroup(heads, t, tk, d, dt, monkeypatch):
+    from intent_attention import dense_attention
+    q, k, v, _ = _qkv(heads + t, (heads,), t, tk, d, d, dt)
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    for causal in (False, True):
+        got = dense_attention(q, k, v, causal=causal)
+        rows = _rows_form(monkeypatch, q, k, v, causal=causal)
+        _check(got, rows.double().cpu().numpy(), dt, f"{dt} {heads}x{t}x{tk}x{d} causal={causal}")
+        # one head in float64
+        n = lambda x: x[heads // 2:heads // 2 + 1].double().cpu().numpy()  # noqa: E731
+        _check(got[heads // 2:heads // 2 + 1], A.dense_attention_masked(n(q), n(k), n(v), causal=causal), dt, "one head")
