@@ -34,6 +34,7 @@
 #include "iak.h"
 #include "iak_internal.h"
 #include "iak_device.h"
+#include "scale_quotient.h"
 
 namespace iak {
 
@@ -96,6 +97,118 @@ __device__ __forceinline__ uint32_t e4m3fn_rne(float v) {
   return sign | code;
 }
 
+// INT4_RESIDUAL codes of a page of finite values that are not all (nearly) zero: false,
+// and nothing written, for any other page. This kernel is bound by its arithmetic
+// (32,771 pages x 128: 81 us in the plain form with its IEEE divisions, where the other
+// precisions take 36 to 41 us for the same traffic; this form 45 to 51), so here pairs of values stay in packed float16 where the arithmetic is
+// float16 anyway, no value is tested for NaN, and adding 1.5 * 2^10 + 8 (float16) or
+// 1.5 * 2^23 + 8 rounds to the integer, ties to even, and leaves code + 8 in the low byte.
+template <int NL>
+__device__ __forceinline__ bool finite_residual_codes(const h8 (&v)[NL], uint32_t (&out)[NL][2], float& s, float& s2) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  typedef float f2v __attribute__((ext_vector_type(2)));
+  us2 m = us2{0, 0};
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const u4 b = __builtin_bit_cast(u4, v[i]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) m = __builtin_elementwise_max(m, __builtin_bit_cast(us2, b[w] & 0x7FFF7FFFu));
+  }
+  const unsigned short am = m[0] > m[1] ? m[0] : m[1];
+  if (__builtin_amdgcn_ballot_w64(am >= 0x7C00u)) return false;
+  s = f16r(wave_max((float)__builtin_bit_cast(_Float16, am), 63) / 127.0f);
+  if (!(s > 0.f)) return false;
+  const float r = 1.0f / s;
+  const _Float16 bias = (_Float16)1544.f, lim = (_Float16)7.f;
+  uint32_t base[NL][4];   // code + 8 of two values, in the low byte of each half
+  float res[NL][8];
+  float ram = 0.f;
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float q[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float x = (float)v[i][2 * w + e], q0 = x * r;
+        q[e] = __builtin_fmaf(__builtin_fmaf(-q0, s, x), r, q0);   // div_by_scale; a zero's sign is not needed
+        asm("" : "+v"(q[e]));   // rounded to float32, then to float16: no mixed-precision fma
+      }
+      const h2 c = __builtin_elementwise_min(
+          __builtin_elementwise_max(__builtin_convertvector((f2v{q[0], q[1]}), h2), (h2{(_Float16)-lim, (_Float16)-lim})),
+          (h2{lim, lim}));
+      const h2 t = c + h2{bias, bias}, code = t - h2{bias, bias};
+      base[i][w] = __builtin_bit_cast(uint32_t, t);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        res[i][2 * w + e] = __builtin_fmaf(-(float)code[e], s, (float)v[i][2 * w + e]);   // code * s is exact
+        ram = fmaxf(ram, fabsf(res[i][2 * w + e]));
+      }
+    }
+  s2 = fmaxf(wave_max(ram, 63) / 127.0f, 1e-8f);
+  const float r2 = 1.0f / s2;
+#pragma unroll
+  for (int i = 0; i < NL; ++i)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      uint32_t z[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        z[e] = __builtin_bit_cast(
+            uint32_t, __builtin_amdgcn_fmed3f(scale_quotient(res[i][4 * k + e], s2, r2), -7.f, 7.f) + 12582920.f);
+      const uint32_t hi = __builtin_amdgcn_perm(z[1], z[0], 0x0C0C0400u) | __builtin_amdgcn_perm(z[3], z[2], 0x04000C0Cu);
+      out[i][k] = __builtin_amdgcn_perm(base[i][2 * k + 1], base[i][2 * k], 0x06040200u) | (hi << 4);
+    }
+  return true;
+}
+
+// INT4_RESIDUAL codes of one page in the plain form, stored: a zero scale's infinities and
+// NaNs, and inf / NaN values, take the IEEE divisions and give code 0. The runs are read
+// again for each pass, so that this rare path holds no registers beside the other
+// (holding its values: 149 registers, three waves per SIMD).
+template <int NL>
+__device__ __forceinline__ void any_residual_codes(const _Float16* src, uint8_t* codes, int step, int lane, float& s,
+                                                   float& s2) {
+  float am = 0.f;
+#pragma unroll 1
+  for (int i = 0; i < NL; ++i) {
+    const h8 v = *reinterpret_cast<const h8*>(src + i * 512 + 8 * lane);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf((float)v[e]));
+  }
+  const float scale = f16r(wave_max(am, 63) / 127.0f);
+  auto base_code = [&](float x) {
+    const float q = f16r(x / scale);
+    return (q != q) ? 0 : (int)__builtin_rintf(fminf(fmaxf(q, -7.f), 7.f));
+  };
+  float ram = 0.f;
+#pragma unroll 1
+  for (int i = 0; i < NL; ++i) {
+    const h8 v = *reinterpret_cast<const h8*>(src + i * 512 + 8 * lane);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = (float)v[e];
+      ram = fmaxf(ram, fabsf(x - (float)base_code(x) * scale));   // float32, as the reference promotes
+    }
+  }
+  s = scale;
+  s2 = fmaxf(wave_max(ram, 63) / 127.0f, 1e-8f);
+#pragma unroll 1
+  for (int i = 0; i < NL; ++i) {
+    const h8 v = *reinterpret_cast<const h8*>(src + i * 512 + 8 * lane);
+    u2 out = u2{0, 0};
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = (float)v[e];
+      const int q1 = base_code(x);
+      const float q = (x - (float)q1 * scale) / s2;
+      const int q2 = (q != q) ? 0 : (int)__builtin_rintf(fminf(fmaxf(q, -7.f), 7.f));
+      out[e / 4] |= (uint32_t)((q1 + 8) | ((q2 + 8) << 4)) << (8 * (e % 4));
+    }
+    *reinterpret_cast<u2*>(codes + i * step) = out;
+  }
+}
+
 // KIND: the precision tag for IAK_QUANT_FAKE_QUANTIZE, or KIND_FUSED / KIND_TRITON
 constexpr int KIND_FUSED = 16, KIND_TRITON = 17;
 
@@ -113,20 +226,38 @@ __global__ __launch_bounds__(256) void quantize_pages_kernel(const iak_quantize_
   const int t0 = lane / LPT;                  // token of run 0; run i holds token t0 + TPL * i
 
   const _Float16* src = reinterpret_cast<const _Float16*>(a.src) + (int64_t)page * PS * D;
+  h8 v[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) v[i] = ld_nt(reinterpret_cast<const h8*>(src + i * 512 + 8 * lane));
+
+  uint8_t* codes = reinterpret_cast<uint8_t*>(a.codes);
+  if constexpr (KIND == IAK_TAG_INT4_RESIDUAL) {
+    uint32_t out[NL][2];
+    float s, s2;
+    codes += (dst * PS + t0) * D + c0;
+    if (finite_residual_codes(v, out, s, s2)) {
+#pragma unroll
+      for (int i = 0; i < NL; ++i) st_nt(reinterpret_cast<u2*>(codes + TPL * i * D), u2{out[i][0], out[i][1]});
+    } else {
+      any_residual_codes<NL>(src, codes, TPL * D, lane, s, s2);
+    }
+    if (lane == 0) {
+      reinterpret_cast<float*>(a.scales)[2 * dst] = s;
+      reinterpret_cast<float*>(a.scales)[2 * dst + 1] = s2;
+    }
+    return;
+  }
+
   float x[NL][8];
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const h8 v = ld_nt(reinterpret_cast<const h8*>(src + i * 512 + 8 * lane));
+  for (int i = 0; i < NL; ++i)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) x[i][e] = (float)v[e];
-  }
+    for (int e = 0; e < 8; ++e) x[i][e] = (float)v[i][e];
   float am = 0.f;
 #pragma unroll
   for (int i = 0; i < NL; ++i)
 #pragma unroll
     for (int e = 0; e < 8; ++e) am = fmaxf(am, fabsf(x[i][e]));
-
-  uint8_t* codes = reinterpret_cast<uint8_t*>(a.codes);
 
   if constexpr (KIND == IAK_TAG_INT4) {
     // group = the lanes of one token whose channels share the group, over all tokens
@@ -158,7 +289,7 @@ __global__ __launch_bounds__(256) void quantize_pages_kernel(const iak_quantize_
   uint32_t out[NL][2];
 #pragma unroll
   for (int i = 0; i < NL; ++i) out[i][0] = out[i][1] = 0;
-  float s = 0.f, s2 = 0.f;
+  float s = 0.f;
 
   if constexpr (KIND == KIND_FUSED) {
     s = f16r(f16r(fmaxf(pam, 1e-6f)) / 127.0f);
@@ -174,13 +305,14 @@ __global__ __launch_bounds__(256) void quantize_pages_kernel(const iak_quantize_
       }
   } else if constexpr (KIND == KIND_TRITON) {
     s = fmaxf(pam, 1e-6f) / 127.0f;
+    const float r = 1.0f / s;   // s = inf gives NaN for x / inf = 0: both code 0
 #pragma unroll
     for (int i = 0; i < NL; ++i)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float q = x[i][e] / s;
-        const float r = (q != q) ? 0.f : fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f);
-        out[i][e / 4] |= ((uint32_t)(int)r & 0xFFu) << (8 * (e % 4));
+        const float q = scale_quotient(x[i][e], s, r);
+        const float c = (q != q) ? 0.f : fminf(fmaxf(__builtin_rintf(q), -127.f), 127.f);
+        out[i][e / 4] |= ((uint32_t)(int)c & 0xFFu) << (8 * (e % 4));
       }
   } else if constexpr (KIND == IAK_TAG_FP8) {
     s = f16r(pam / 127.0f);
@@ -219,45 +351,14 @@ __global__ __launch_bounds__(256) void quantize_pages_kernel(const iak_quantize_
         const float r = (q != q) ? 0.f : __builtin_rintf(fminf(fmaxf(q, -127.f), 127.f));
         out[i][e / 4] |= ((uint32_t)(int)r & 0xFFu) << (8 * (e % 4));
       }
-  } else {   // INT4_RESIDUAL
-    s = f16r(pam / 127.0f);
-    float res[NL][8];
-    int q1[NL][8];
-    float ram = 0.f;
-    float qs[NL][8];
-    scale_quotients(x, s, qs);
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float q = f16r(qs[i][e]);
-        q1[i][e] = (q != q) ? 0 : (int)__builtin_rintf(fminf(fmaxf(q, -7.f), 7.f));
-        res[i][e] = x[i][e] - (float)q1[i][e] * s;      // float32, as the reference promotes
-        ram = fmaxf(ram, fabsf(res[i][e]));
-      }
-    s2 = fmaxf(wave_max(ram, 63) / 127.0f, 1e-8f);
-#pragma unroll
-    for (int i = 0; i < NL; ++i)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float q = res[i][e] / s2;
-        const int q2 = (q != q) ? 0 : (int)__builtin_rintf(fminf(fmaxf(q, -7.f), 7.f));
-        out[i][e / 4] |= (uint32_t)((q1[i][e] + 8) | ((q2 + 8) << 4)) << (8 * (e % 4));
-      }
   }
 
 #pragma unroll
   for (int i = 0; i < NL; ++i) {
-    u2 v;
-    v[0] = out[i][0];
-    v[1] = out[i][1];
-    st_nt(reinterpret_cast<u2*>(codes + (dst * PS + t0 + TPL * i) * D + c0), v);
+    st_nt(reinterpret_cast<u2*>(codes + (dst * PS + t0 + TPL * i) * D + c0), u2{out[i][0], out[i][1]});
   }
   if (lane == 0) {
-    if (KIND == IAK_TAG_INT4_RESIDUAL) {
-      reinterpret_cast<float*>(a.scales)[2 * dst] = s;
-      reinterpret_cast<float*>(a.scales)[2 * dst + 1] = s2;
-    } else if (a.scale_dtype == IAK_DTYPE_F32) {
+    if (a.scale_dtype == IAK_DTYPE_F32) {
       reinterpret_cast<float*>(a.scales)[dst] = s;
     } else {
       reinterpret_cast<_Float16*>(a.scales)[dst] = (_Float16)s;
