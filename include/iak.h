@@ -43,6 +43,7 @@
  *                               kv_memory_manager.py:233-252, _read_page_data :286-296, set_page_format
  *                               :268-284 (demote_cold_pages :350-362, promote_hot_pages :364-377)
  *   iak_prefetch_pages          launch_prefetch_pages() prefetch.py:183-261 (its Triton kernel :111-170)
+ *   iak_mla_project             the projection by W_VO in mla_decode_triton() triton_mla_decode.py:146-151
  *   iak_dense_attention         dense_attention() reference.py:16-45 (causal, mask, original_kv_positions),
  *                               under semantic_block_attention() reference.py:81-129 and
  *                               intent_quant_attention_reference() intent_quant_attention.py:20-119
@@ -505,6 +506,20 @@ iak_status iak_mla_decode_rows_workspace(const iak_mla_rows_args* args, size_t* 
 
 iak_status iak_mla_decode_rows(const iak_mla_rows_args* args, void* workspace, size_t workspace_bytes,
                                void* stream);
+
+/* The projection of those contexts by W_VO in float32 (triton_mla_decode.py:146-151), for a
+ * decode step's rows: out[row, n] = sum over k of context[row, k] w[k, n].
+ *   context [rows, latent_dim] float32, contiguous, 16-byte aligned; latent_dim a multiple of 8
+ *   w       [latent_dim, d_out] (w_dtype), element row stride w_stride; d_out a multiple of 32
+ *   out     [rows, d_out] (out_dtype), contiguous (written) */
+typedef struct {
+  int32_t rows, latent_dim, d_out;
+  const float* context;
+  const void* w; int32_t w_dtype; int64_t w_stride;
+  void* out; int32_t out_dtype;
+} iak_mla_project_args;
+
+iak_status iak_mla_project(const iak_mla_project_args* args, void* stream);
 
 /* Dense softmax attention of the reference's dense_attention() (reference.py:16-45)
  * in float32: for each (batch, query) row i,

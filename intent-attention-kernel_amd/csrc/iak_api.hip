@@ -370,6 +370,7 @@ iak_status scratch_address(int dev, void** out) {
 namespace iak {
 hipError_t launch_mla_rows(const iak_mla_rows_args& a, void* workspace, hipStream_t stream);   // mla_rows.hip
 hipError_t launch_mla_few_heads(const MArgs& m, hipStream_t stream, hipEvent_t ev_begin, hipEvent_t ev_end);   // mla_decode.hip; HG = groups of 16 heads
+hipError_t launch_mla_project(const iak_mla_project_args& a, hipStream_t stream);             // mla_rows.hip
 size_t mla_rows_workspace(const iak_mla_rows_args& a);                                      // mla_rows.hip
 hipError_t launch_fake_quant_blocks(const iak_fake_quant_blocks_args& a, void* workspace,
                                     hipStream_t stream);                    // fake_quant.hip
@@ -788,6 +789,24 @@ iak_status iak_mla_decode_rows(const iak_mla_rows_args* a, void* workspace, size
     if (!aligned16(workspace)) return fail(IAK_EINVAL, "workspace must be 16-byte aligned");
   }
   const hipError_t e = iak::launch_mla_rows(*a, workspace, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(IAK_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
+  return IAK_OK;
+}
+
+iak_status iak_mla_project(const iak_mla_project_args* a, void* stream) {
+  if (!a) return fail(IAK_EINVAL, "args is NULL");
+  if (a->rows < 0 || a->latent_dim <= 0 || a->d_out < 0)
+    return fail(IAK_EINVAL, "bad size (rows=%d, latent_dim=%d, d_out=%d)", a->rows, a->latent_dim, a->d_out);
+  if (a->latent_dim % 8 || a->d_out % 32)
+    return fail(IAK_ENOTSUP, "latent_dim %d / d_out %d is not supported (multiples of 8 / 32)", a->latent_dim, a->d_out);
+  if (a->rows > 32 * 65535) return fail(IAK_ENOTSUP, "rows = %d is not supported (at most %d)", a->rows, 32 * 65535);
+  if (a->w_dtype < 0 || a->w_dtype > 2) return fail(IAK_EINVAL, "unknown w dtype %d", a->w_dtype);
+  if (a->out_dtype < 0 || a->out_dtype > 2) return fail(IAK_EINVAL, "unknown out dtype %d", a->out_dtype);
+  if (a->rows == 0 || a->d_out == 0) return IAK_OK;
+  if (!a->context || !a->w || !a->out) return fail(IAK_EINVAL, "context/w/out is NULL");
+  if (!aligned16(a->context)) return fail(IAK_EINVAL, "context must be 16-byte aligned");
+  if (a->w_stride < 0) return fail(IAK_EINVAL, "negative stride %lld", (long long)a->w_stride);
+  const hipError_t e = iak::launch_mla_project(*a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(IAK_EHIP, "kernel launch failed: %s", hipGetErrorString(e));
   return IAK_OK;
 }

@@ -343,6 +343,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void mla_rows_merge_kernel(const iak
 }
 
 #include "mla_rows_matrix.h"
+#include "mla_project.h"
 
 // MAXW: the most waves per workgroup whose registers and LDS fit
 template <typename T, int NPL, int KEYS, int MAXW, int R>
@@ -486,6 +487,14 @@ hipError_t launch_mla_rows(const iak_mla_rows_args& a, void* workspace, hipStrea
   if (a.latent_dtype == IAK_DTYPE_F32) launch_typed<float>(a, sp, stream);
   else if (a.latent_dtype == IAK_DTYPE_F16) launch_typed<_Float16>(a, sp, stream);
   else launch_typed<bf16_bits>(a, sp, stream);
+  return hipGetLastError();
+}
+
+hipError_t launch_mla_project(const iak_mla_project_args& a, hipStream_t stream) {
+  const dim3 grid((unsigned)(a.d_out / PJ_COLS), (unsigned)((a.rows + PJ_ROWS - 1) / PJ_ROWS)), block(64 * PJ_WAVES);
+  if (a.w_dtype == IAK_DTYPE_F32) hipLaunchKernelGGL(mla_project_kernel<float>, grid, block, 0, stream, a);
+  else if (a.w_dtype == IAK_DTYPE_F16) hipLaunchKernelGGL(mla_project_kernel<_Float16>, grid, block, 0, stream, a);
+  else hipLaunchKernelGGL(mla_project_kernel<bf16_bits>, grid, block, 0, stream, a);
   return hipGetLastError();
 }
 

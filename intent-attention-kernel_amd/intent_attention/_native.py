@@ -145,6 +145,17 @@ class MlaRowsArgs(ctypes.Structure):
     ]
 
 
+class MlaProjectArgs(ctypes.Structure):
+    """Mirror of ``iak_mla_project_args`` (include/iak.h)."""
+
+    _fields_ = [
+        ("rows", c_i32), ("latent_dim", c_i32), ("d_out", c_i32),
+        ("context", c_void_p),
+        ("w", c_void_p), ("w_dtype", c_i32), ("w_stride", c_i64),
+        ("out", c_void_p), ("out_dtype", c_i32),
+    ]
+
+
 FQ_FP16, FQ_FP8, FQ_INT8, FQ_INT4, FQ_INT4_RESIDUAL, FQ_SKIP = 0, 1, 2, 3, 4, 5   # IAK_FQ_*
 
 
@@ -183,7 +194,7 @@ EXPORTED = ("iak_abi_version", "iak_status_string", "iak_last_error",
             "iak_mla_decode_workspace", "iak_mla_decode", "iak_quantize_pages",
             "iak_build_page_tables", "iak_paged_decode_timed", "iak_mla_decode_timed",
             "iak_paged_decode_noalloc", "iak_transcode_pages", "iak_prefetch_pages", "iak_paged_decode_plan",
-            "iak_mla_decode_rows", "iak_pack_page_descriptors",
+            "iak_mla_decode_rows", "iak_mla_project", "iak_pack_page_descriptors",
             "iak_pack_entry_records", "iak_dense_attention", "iak_dense_attention_indexed", "iak_dense_attention_workspace",
             "iak_mla_decode_rows_workspace", "iak_fake_quant_blocks",
             "iak_fake_quant_blocks_workspace", "iak_timing_event_create", "iak_timing_event_record",
@@ -241,6 +252,8 @@ def load() -> ctypes.CDLL:
     lib.iak_prefetch_pages.restype = ctypes.c_int
     lib.iak_prefetch_pages.argtypes = [ctypes.POINTER(PrefetchArgs), c_void_p]
     lib.iak_build_page_tables.restype = ctypes.c_int
+    lib.iak_mla_project.restype = ctypes.c_int
+    lib.iak_mla_project.argtypes = [ctypes.POINTER(MlaProjectArgs), c_void_p]
     lib.iak_mla_decode_rows.restype = ctypes.c_int
     lib.iak_mla_decode_rows.argtypes = [ctypes.POINTER(MlaRowsArgs), c_void_p, ctypes.c_size_t, c_void_p]
     lib.iak_timing_event_create.restype = ctypes.c_int
@@ -379,6 +392,10 @@ def mla_decode_rows_workspace(args: MlaRowsArgs) -> int:
 
 def mla_decode_rows(args: MlaRowsArgs, stream: int, workspace: int = 0, workspace_bytes: int = 0) -> None:
     check(load().iak_mla_decode_rows(ctypes.byref(args), workspace or None, workspace_bytes, stream or None))
+
+
+def mla_project(args: MlaProjectArgs, stream: int) -> None:
+    check(load().iak_mla_project(ctypes.byref(args), stream or None))
 
 
 def build_page_tables(args: PageTableArgs, stream: int) -> None:

@@ -10,7 +10,7 @@ the context is projected by ``W_VO_fused``; zeros when the table is empty.
 The latent context runs on libiak's ``iak_mla_decode_rows`` in the reference's
 arithmetic: float32 products and sums over the inputs as given (float32,
 float16 or bfloat16, read in place), any ``page_size``, any ``d_c`` up to 1,024
-in one launch. The projection is one float32 GEMM. (The paged serving path,
+in one launch. The projection is a float32 product over W as it is stored. (The paged serving path,
 ``mla_core.mla_paged_decode``, is the MFMA kernel over f16 / FP8 / INT8 latent
 pools.) Host tensors raise RuntimeError: there is no CPU path in this package.
 """
@@ -19,12 +19,16 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd import forward_ad as _fwd_ad
 
 from . import _native as N
 from .decode_core import current_stream_handle, require_device
 
 _DT = {torch.float32: N.DTYPE_F32, torch.float16: N.DTYPE_F16, torch.bfloat16: N.DTYPE_BF16}
 MAX_LATENT = 1024
+# the projection kernel reads W once per 32 rows: 128 rows x 576 x 4,096 11.0 us against 24.7
+# for W.float() and a GEMM, 192 rows 15.2 / 26.7, 256 rows 19.2 to 20.3 / 25
+MAX_PROJECT_ROWS = 128
 
 
 def is_triton_available() -> bool:
@@ -80,6 +84,19 @@ def mla_latent_context(q_absorb: torch.Tensor, C: torch.Tensor, page_table: torc
     return ctx
 
 
+def _projects(ctx: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the projection runs on libiak's kernel, which reads W as it is stored: up to
+    MAX_PROJECT_ROWS rows over whole 8 x 32 pieces of a row-major W. Wherever torch would do
+    more than multiply (a W that is differentiated, in either mode, mapped over or a
+    subclass; autocast), and for more rows, torch's float32 GEMM over W.float() keeps it."""
+    return (type(w) in (torch.Tensor, torch.nn.Parameter) and w.dtype in _DT
+            and 0 < ctx.shape[0] * ctx.shape[1] <= MAX_PROJECT_ROWS
+            and not w.is_neg() and w.stride(1) == 1 and w.shape[0] % 8 == 0 and w.shape[1] % 32 == 0 and w.shape[1] > 0
+            and not (w.requires_grad and torch.is_grad_enabled()) and _fwd_ad._current_level < 0
+            and not torch._C._functorch.is_functorch_wrapped_tensor(w)
+            and not torch.is_autocast_enabled(ctx.device.type))
+
+
 def mla_decode_triton(q_absorb: torch.Tensor, C: torch.Tensor, W_VO_fused: torch.Tensor,
                       page_table: torch.Tensor, page_size: int = 64) -> torch.Tensor:
     """MLA decode over page-table-selected latent pages (triton_mla_decode.py:110-152).
@@ -91,4 +108,14 @@ def mla_decode_triton(q_absorb: torch.Tensor, C: torch.Tensor, W_VO_fused: torch
     if W_VO_fused.dim() != 2 or W_VO_fused.shape[0] != q_absorb.shape[2]:
         raise ValueError(f"W_VO_fused must be [d_c, d_out], got {tuple(W_VO_fused.shape)}")
     ctx = mla_latent_context(q_absorb, C, page_table, page_size)
-    return (ctx @ W_VO_fused.float()).to(q_absorb.dtype)
+    if not _projects(ctx, W_VO_fused):
+        return (ctx @ W_VO_fused.float()).to(q_absorb.dtype)
+    batch, q_len, d_c = ctx.shape
+    out = torch.empty(batch, q_len, W_VO_fused.shape[1], dtype=q_absorb.dtype, device=ctx.device)
+    a = N.MlaProjectArgs()
+    a.rows, a.latent_dim, a.d_out = batch * q_len, d_c, W_VO_fused.shape[1]
+    a.context = ctx.data_ptr()
+    a.w, a.w_dtype, a.w_stride = W_VO_fused.data_ptr(), _DT[W_VO_fused.dtype], W_VO_fused.stride(0)
+    a.out, a.out_dtype = out.data_ptr(), _DT[out.dtype]
+    N.mla_project(a, current_stream_handle(ctx.device))
+    return out

@@ -221,6 +221,7 @@ void invalid_launches() {
   }
   count(iak_dense_attention(nullptr, nullptr, 0, nullptr));
   count(iak_dense_attention_indexed(nullptr, nullptr, nullptr, 0, nullptr));
+  count(iak_mla_project(nullptr, nullptr));
 
   // workspace sizes of random and of valid shapes (host queries), and a split
   // shape with a workspace one byte short (rejected before the launch)
