@@ -338,8 +338,8 @@ __device__ __forceinline__ float block_reduce(float v, float* red) {
 // (splits <= MAX_SPLITS). The split weights go to the LDS; each context dim is
 // then summed over the splits by G thread groups (G = 256 / dims rounded up to
 // 64), each over every G-th split, with eight independent loads in flight.
-// FLAGS: the partials come from dense_matrix_kernel with key-tile flags; a row of
-// a flagged batch entry is computed again from its inputs.
+// FLAGS: the partials come from dense_matrix_kernel; a row of a batch entry with a
+// flagged key tile is computed again from its inputs.
 template <typename T, bool FLAGS>
 __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseArgs a,
                                                                     const DenseSplit sp, const MatrixPlan mp) {
@@ -549,11 +549,6 @@ MatrixPlan matrix_plan(const DenseArgs& a, const MatrixShape& s) {
   return mp;
 }
 
-// key-tile flags are needed where a weight is split or tiles are skipped
-bool matrix_flags(const DenseArgs& a, const MatrixPlan& mp) {
-  return a.dtype != IAK_DTYPE_F32 || mp.skip;
-}
-
 size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
   if (mp.splits <= 1) return 0;
   return ((size_t)mp.accoff + (size_t)a.batch * a.q_len * mp.splits * (size_t)a.v_dim) * sizeof(float);
@@ -561,9 +556,7 @@ size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
 
 size_t matrix_workspace(const DenseArgs& a) {
   const MatrixPlan mp = matrix_plan(a, matrix_shape(a));
-  const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * mp.waves * sizeof(int32_t) : 0;
-  const size_t total = matrix_partial_bytes(a, mp) + flags;
-  return total ? total : 16;   // a workspace at all says that the form may run
+  return matrix_partial_bytes(a, mp) + (size_t)a.batch * mp.nt * mp.waves * sizeof(int32_t);
 }
 
 template <typename T, int DP, int QW, int KW, int BKW>
@@ -596,8 +589,7 @@ void launch_matrix(const DenseArgs& a, void* workspace, hipStream_t stream) {
   const MatrixShape s = matrix_shape(a);
   MatrixPlan mp = matrix_plan(a, s);
   mp.ws = static_cast<float*>(workspace);
-  const bool flags = matrix_flags(a, mp);
-  if (flags) mp.flags = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + matrix_partial_bytes(a, mp));
+  mp.flags = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + matrix_partial_bytes(a, mp));
   if (s.dp == 64) launch_matrix_dims<T, 64>(a, s, mp, stream);
   else if (s.dp == 128) launch_matrix_dims<T, 128>(a, s, mp, stream);
   if constexpr (sizeof(T) == 2) {
@@ -609,11 +601,8 @@ void launch_matrix(const DenseArgs& a, void* workspace, hipStream_t stream) {
   if (mp.splits > 1) {
     const bool gen = a.mask || a.causal == IAK_CAUSAL_POSITIONS;
     const DenseSplit sp{mp.splits, mp.chunk, mp.ws, mp.accoff, gen ? 0 : 1};
-    if (flags)
-      hipLaunchKernelGGL((dense_merge_kernel<T, true>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
-    else
-      hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
-  } else if (flags) {
+    hipLaunchKernelGGL((dense_merge_kernel<T, true>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
+  } else {
     const int64_t per = a.batch < 256 ? (256 + a.batch - 1) / a.batch : 1;
     hipLaunchKernelGGL(dense_fixup_kernel<T>, dim3((unsigned)(a.batch * per)), dim3(256), 0, stream, a, mp);
   }

@@ -24,8 +24,10 @@
 // carries 22 bits or more (float16: two parts of p * 2^7, bfloat16: three),
 // one matrix instruction per part. float32 inputs: v_mfma_f32_32x32x2_f32.
 //
-// Non-finite values. Two shortcuts would answer differently from the plain sum
-// for them: a split weight times an infinite V (inf * 0 in the low part), and
+// Non-finite and large values. Four shortcuts would answer differently from the plain
+// sum for them: a split weight times an infinite V (inf * 0 in the low part); the
+// rows that fill up a range's last tile, which repeat its last key with weight 0
+// (0 * inf); the lagging maximum, whose weights of up to 2^8 overflow on a finite V; and
 // causal tiles past the diagonal, which are not visited (a NaN or an
 // overflowing score there makes its row NaN, an infinite V a zero weight's
 // product NaN). Each key tile is therefore checked once, by one of the
@@ -55,7 +57,7 @@ struct MatrixPlan {
   int64_t accoff;  // offset of the partial contexts in ws (floats)
   float* ws;       // splits > 1: the partials
   int waves;       // waves of a workgroup
-  int32_t* flags;  // [batch][nt][waves], or null (nothing to check)
+  int32_t* flags;  // [batch][nt][waves]
 };
 
 template <typename T> struct MxElem;   // operand vector of 16 bytes, matrix product, parts of a weight
@@ -311,7 +313,6 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
     if (lane == 0) mp.flags[((int64_t)b * mp.nt + lo / BK + t) * (QW * KW) + w] = any ? 1 : 0;
   };
   auto checks = [&](int t) {
-    if (!mp.flags) return false;
     const int g = lo / BK + t;
     if (!mp.skip) return g % mp.nq == qt;
     const int64_t own = (int64_t)g * BK / C::BQ;      // the first query tile that visits it
@@ -525,7 +526,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
     if (tiles > 0) {
       look_up(0);
       load_k();
-      if (mp.flags) bad = large(kr);
+      bad = checks(0) && large(kr);
       store_k(0);
       load_v();
       if (tiles > 1) look_up(1);
@@ -539,7 +540,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
       if (seen(t)) scores(t, 0);
       sync();   // its keys are read
       if (more) {
-        if (mp.flags) bad = large(kr);
+        bad = checks(t + 1) && large(kr);
         store_k(0);
         load_v();
         if (t + 2 < tiles) look_up(t + 2);
@@ -583,7 +584,7 @@ void dense_matrix_kernel(const DenseArgs a, const MatrixPlan mp) {
     }
   }
   // key tiles that no query tile visits (keys past the last row's diagonal): checked here
-  if (mp.flags && mp.skip) {
+  if (mp.skip) {
     const int all = hi > lo ? (hi - lo + BK - 1) / BK : 0;
     for (int t = 0; t < all; ++t) {
       const int64_t g = lo / BK + t;

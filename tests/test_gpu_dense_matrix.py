@@ -175,3 +175,37 @@ def test_waves_per_workgroup(heads, t, tk, d, dt, monkeypatch):
         # one head in float64
         n = lambda x: x[heads // 2:heads // 2 + 1].double().cpu().numpy()  # noqa: E731
         _check(got[heads // 2:heads // 2 + 1], A.dense_attention_masked(n(q), n(k), n(v), causal=causal), dt, "one head")
+
+
+# key counts one short of a 32- or 128-key tile, one past it, and whole tiles; the wave shapes of
+# few, some and many query rows, keys split over workgroups (2 and 8 heads) and not (300)
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("heads,tq,tk", [(8, 8, 1055), (2, 40, 1025), (2, 128, 1057), (300, 8, 159), (300, 8, 161),
+                                         (300, 33, 65), (300, 130, 33)])
+def test_special_values_in_the_last_key(heads, tq, tk, dt, monkeypatch):
+    """The last key's row stands in for the keys that fill up its tile: whatever it holds, the
+    result is the row form's. Its score is up to 2^7 above the others', as far as the
+    running maximum may lag, so a large finite value must not overflow on the way either."""
+    from intent_attention import BlockLayout, BlockPolicy, SemanticBlock, dense_attention, semantic_block_attention
+    q, k, v, g = _qkv(heads + tk, (heads,), tq, tk, 64, 64, dt)
+    q[..., 0], k[:, :-1] = 4.0, k[:, :-1] * 0.1
+    k[:, -1] = 0.0
+    k[:, -1, 0] = 9.0                                  # 4 * 9 / 8 log2(e) = 6.5
+    big = 60000.0 if dt == "f16" else 1e37
+    mask = torch.zeros(tq, tk).to(DT[dt])
+    mask[:, 5] = float("-inf")
+    pos = torch.arange(tk)
+    layout = BlockLayout([SemanticBlock("a", 0, tk, BlockPolicy.ALWAYS)])
+    forms = [dict(), dict(mask=mask.cuda()), dict(causal=True, original_kv_positions=pos.flip(0).cuda()), dict(causal=True)]
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    for value in (np.inf, -np.inf, np.nan, big, -big):
+        v[0, -1, 3], v[1, -1, :] = value, abs(value)
+        for i, kw in enumerate(forms + [None]):
+            want = _rows_form(monkeypatch, q, k, v, **(kw or {}))
+            got = semantic_block_attention(q, k, v, layout) if kw is None else dense_attention(q, k, v, **kw)
+            what = f"{value} form {i}"
+            for f in (torch.isnan, torch.isposinf, torch.isneginf):
+                assert torch.equal(f(got), f(want)), what
+            live = torch.isfinite(want)
+            scale = want[live].double().abs().clamp(min=1)
+            assert float(((got[live].double() - want[live].double()) / scale).abs().max()) <= 2 * TOL[dt], what
