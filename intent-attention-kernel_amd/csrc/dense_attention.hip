@@ -20,8 +20,9 @@
 //
 // Selected tokens (kv_index) are read where they lie: the gathered K and V of 3,072 of
 // 4,096 tokens x 8 heads x 64 in float32 took two launches of 9 us and a pass over both,
-// the index in the kernel costs nothing that shows (blocks through
-// semantic_block_attention 170 -> 50 us with the index uploaded without a wait).
+// the index costs the kernels that read it no time that shows (blocks through
+// semantic_block_attention 170 -> 50 us with the index uploaded without a wait); the
+// others are compiled without it (dense_row).
 //
 // Work split. A (batch, query) row's keys go to `splits` workgroups of
 // consecutive key ranges (`chunk` keys each); splits > 1 only when the caller
@@ -134,7 +135,10 @@ struct DenseSplit {
 // T: element type of q, k, v and out; NPL: dims per lane (head_dim and v_dim
 // are at most 64 * NPL); KEYS keys per wave and step; WAVES waves per workgroup.
 // `item` = row * splits + split, row = b * q_len + i; `items` of them in all.
-template <typename T, int NPL, int KEYS, int WAVES>
+// INDEXED: kv_index is given (a test of it per step cost the others 5 %: 512 rows x 4,096
+// keys x 128 in float16 229 / 241 us; between the loads, 1,024 rows x 1,000 keys x
+// 1,000 457 / 830 us)
+template <typename T, int NPL, int KEYS, int WAVES, bool INDEXED>
 __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& sp, int64_t item,
                                           int64_t items) {
   __shared__ float part_acc[WAVES][64 * NPL];
@@ -178,7 +182,7 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& 
 #pragma unroll
     for (int u = 0; u < KEYS; ++u) {
       const int jc = j0 + u < hi ? j0 + u : hi - 1;
-      const int64_t at = a.kv_index ? a.kv_index[jc] : jc;   // wave-uniform
+      const int64_t at = INDEXED ? a.kv_index[jc] : jc;   // wave-uniform
       const T* kr = kbase + at * a.k_stride_t;
       const T* vr = vbase + at * a.v_stride_t;
 #pragma unroll
@@ -306,10 +310,18 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& 
   }
 }
 
+// the same, whether kv_index is given or not
 template <typename T, int NPL, int KEYS, int WAVES>
+__device__ __forceinline__ void dense_row_any(const DenseArgs& a, int64_t row) {
+  const DenseSplit one{1, a.kv_len, nullptr, 0, 0};
+  if (a.kv_index) dense_row<T, NPL, KEYS, WAVES, true>(a, one, row, 0);
+  else dense_row<T, NPL, KEYS, WAVES, false>(a, one, row, 0);
+}
+
+template <typename T, int NPL, int KEYS, int WAVES, bool INDEXED>
 __global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const DenseArgs a,
                                                                       const DenseSplit sp) {
-  dense_row<T, NPL, KEYS, WAVES>(a, sp, blockIdx.x, gridDim.x);
+  dense_row<T, NPL, KEYS, WAVES, INDEXED>(a, sp, blockIdx.x, gridDim.x);
 }
 
 #include "dense_matrix.h"
@@ -351,7 +363,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
   const int i = (int)(row - b * a.q_len);
   if constexpr (FLAGS) {
     if (mx_flagged(mp, b)) {
-      dense_row<T, MX_MAX_DIM / 64, 2, MERGE_THREADS / 64>(a, DenseSplit{1, a.kv_len, nullptr, 0, 0}, row, 0);
+      dense_row_any<T, MX_MAX_DIM / 64, 2, MERGE_THREADS / 64>(a, row);
       return;
     }
   }
@@ -408,32 +420,32 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
 
 // MAXW: the most waves per workgroup whose registers and LDS fit (16 waves of
 // a 1,024-thread workgroup get 128 VGPRs each)
-template <typename T, int NPL, int KEYS, int MAXW>
+template <typename T, int NPL, int KEYS, int MAXW, bool INDEXED>
 void launch_items(const DenseArgs& a, const DenseSplit& sp, int64_t items, hipStream_t stream) {
   // waves per workgroup: about 4,096 waves in the grid (16 per CU), between 4 and MAXW
   const int64_t want = (4096 + items - 1) / items;
   const dim3 grid((unsigned)items);
   if (MAXW >= 16 && want >= 16)
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, MAXW >= 16 ? 16 : 4>), grid, dim3(1024), 0, stream,
-                       a, sp);
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, MAXW >= 16 ? 16 : 4, INDEXED>), grid, dim3(1024), 0,
+                       stream, a, sp);
   else if (want >= 8)
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 8>), grid, dim3(512), 0, stream, a, sp);
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 8, INDEXED>), grid, dim3(512), 0, stream, a, sp);
   else
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 4>), grid, dim3(256), 0, stream, a, sp);
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 4, INDEXED>), grid, dim3(256), 0, stream, a, sp);
 }
 
-template <typename T>
+template <typename T, bool INDEXED>
 void launch_rows(const DenseArgs& a, const DenseSplit& sp, hipStream_t stream) {
   const int64_t rows = (int64_t)a.batch * a.q_len;
   const int64_t items = rows * sp.splits;
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
   const int npl = (width + 63) / 64;
   // keys per step: 2 * KEYS * NPL registers of K and V in flight per lane
-  if (npl <= 1) launch_items<T, 1, 8, 16>(a, sp, items, stream);
-  else if (npl <= 2) launch_items<T, 2, 8, 16>(a, sp, items, stream);
-  else if (npl <= 4) launch_items<T, 4, 4, 16>(a, sp, items, stream);
-  else if (npl <= 8) launch_items<T, 8, 4, 8>(a, sp, items, stream);
-  else launch_items<T, 16, 2, 8>(a, sp, items, stream);
+  if (npl <= 1) launch_items<T, 1, 8, 16, INDEXED>(a, sp, items, stream);
+  else if (npl <= 2) launch_items<T, 2, 8, 16, INDEXED>(a, sp, items, stream);
+  else if (npl <= 4) launch_items<T, 4, 4, 16, INDEXED>(a, sp, items, stream);
+  else if (npl <= 8) launch_items<T, 8, 4, 8, INDEXED>(a, sp, items, stream);
+  else launch_items<T, 16, 2, 8, INDEXED>(a, sp, items, stream);
   if (sp.splits > 1)
     hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp,
                        MatrixPlan{});
@@ -614,7 +626,8 @@ void launch_typed(const DenseArgs& a, void* workspace, hipStream_t stream) {
   DenseSplit sp = split_plan(a);
   if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr, 0, 0};
   sp.ws = static_cast<float*>(workspace);
-  launch_rows<T>(a, sp, stream);
+  if (a.kv_index) launch_rows<T, true>(a, sp, stream);
+  else launch_rows<T, false>(a, sp, stream);
 }
 
 }  // namespace

@@ -700,9 +700,8 @@ template <typename T>
 __global__ __launch_bounds__(256) void dense_fixup_kernel(const DenseArgs a, const MatrixPlan mp) {
   const int64_t b = blockIdx.x % (unsigned)a.batch, first = blockIdx.x / (unsigned)a.batch;
   if (!mx_flagged(mp, b)) return;
-  const DenseSplit one{1, a.kv_len, nullptr, 0, 0};
   for (int64_t i = first; i < a.q_len; i += gridDim.x / (unsigned)a.batch) {
-    dense_row<T, MX_MAX_DIM / 64, 2, 4>(a, one, b * a.q_len + i, 0);
+    dense_row_any<T, MX_MAX_DIM / 64, 2, 4>(a, b * a.q_len + i);
     __syncthreads();   // its LDS is free for the next row
   }
 }
