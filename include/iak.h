@@ -542,10 +542,12 @@ iak_status iak_mla_project(const iak_mla_project_args* args, void* stream);
  * many keys splits each row's keys over several workgroups and merges their
  * partials in a second kernel; it must then hold iak_dense_attention_workspace()
  * bytes (16-byte aligned; 0 bytes means neither applies and the workspace is
- * unused). Without it every row runs in one workgroup. The results agree to
+ * unused; IAK_DENSE_NO_SCRATCH bytes means that the matrix cores do without one: any 16
+ * bytes of device memory, which stay as they are, ask for them). Without it every row runs in one workgroup. The results agree to
  * float32 rounding of the summation order, NaN and infinities included. Calls
  * that share a workspace on different streams race. */
 enum { IAK_MASK_BOOL = 3 };
+enum { IAK_DENSE_NO_SCRATCH = 16 };
 enum { IAK_CAUSAL_NONE = 0, IAK_CAUSAL_TRIU = 1, IAK_CAUSAL_POSITIONS = 2 };
 typedef struct {
   int32_t batch, q_len, kv_len, head_dim, v_dim, dtype;

@@ -41,6 +41,7 @@
 #include <stdint.h>
 
 #include <cmath>
+#include <type_traits>
 
 #include "iak.h"
 #include "iak_device.h"
@@ -97,7 +98,7 @@ struct DenseArgs : iak_dense_attention_args {
 // the mask values of keys j0 .. j0 + KEYS - 1 of one query row (indices
 // clamped to the range's last key `last`)
 template <typename M, int KEYS>
-__device__ __forceinline__ void step_mask(const DenseArgs& a, int64_t mb, int j0, int last,
+__device__ __forceinline__ void step_mask(const iak_dense_attention_args& a, int64_t mb, int j0, int last,
                                           float* madd) {
 #pragma unroll
   for (int u = 0; u < KEYS; ++u) {
@@ -128,19 +129,17 @@ struct DenseSplit {
   int splits;   // workgroups per row
   int chunk;    // keys per workgroup (the last may have fewer)
   float* ws;    // splits > 1: [rows * splits] max, [rows * splits] denominator, [rows * splits, v_dim] context
-  int64_t accoff;   // offset of the contexts in ws (floats)
-  int log2;         // the maxima are in the exp2 domain
 };
 
 // T: element type of q, k, v and out; NPL: dims per lane (head_dim and v_dim
 // are at most 64 * NPL); KEYS keys per wave and step; WAVES waves per workgroup.
 // `item` = row * splits + split, row = b * q_len + i; `items` of them in all.
-// INDEXED: kv_index is given (a test of it per step cost the others 5 %: 512 rows x 4,096
+// INDEX: whether kv_index is given, or ANY_INDEX (a test of it per step cost the others 5 %: 512 rows x 4,096
 // keys x 128 in float16 229 / 241 us; between the loads, 1,024 rows x 1,000 keys x
 // 1,000 457 / 830 us)
-template <typename T, int NPL, int KEYS, int WAVES, bool INDEXED>
-__device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& sp, int64_t item,
-                                          int64_t items) {
+constexpr int ANY_INDEX = 2;
+template <typename T, int NPL, int KEYS, int WAVES, int INDEX, typename Args>
+__device__ __forceinline__ void dense_row(const Args& a, const DenseSplit& sp, int64_t item, int64_t items) {
   __shared__ float part_acc[WAVES][64 * NPL];
   __shared__ float part_m[WAVES], part_l[WAVES];
   const int lane = threadIdx.x & 63;
@@ -182,7 +181,9 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& 
 #pragma unroll
     for (int u = 0; u < KEYS; ++u) {
       const int jc = j0 + u < hi ? j0 + u : hi - 1;
-      const int64_t at = INDEXED ? a.kv_index[jc] : jc;   // wave-uniform
+      int64_t at = jc;   // wave-uniform
+      if constexpr (INDEX == 1) at = a.kv_index[jc];
+      else if constexpr (INDEX == ANY_INDEX) at = a.kv_index ? a.kv_index[jc] : jc;
       const T* kr = kbase + at * a.k_stride_t;
       const T* vr = vbase + at * a.v_stride_t;
 #pragma unroll
@@ -290,7 +291,7 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& 
       sp.ws[item] = M;
       sp.ws[items + item] = L;
     }
-    float* wacc = sp.ws + sp.accoff + item * a.v_dim;
+    float* wacc = sp.ws + 2 * items + item * a.v_dim;
     for (int d = threadIdx.x; d < a.v_dim; d += 64 * WAVES) {
       float A = 0.f;
 #pragma unroll
@@ -310,18 +311,10 @@ __device__ __forceinline__ void dense_row(const DenseArgs& a, const DenseSplit& 
   }
 }
 
-// the same, whether kv_index is given or not
-template <typename T, int NPL, int KEYS, int WAVES>
-__device__ __forceinline__ void dense_row_any(const DenseArgs& a, int64_t row) {
-  const DenseSplit one{1, a.kv_len, nullptr, 0, 0};
-  if (a.kv_index) dense_row<T, NPL, KEYS, WAVES, true>(a, one, row, 0);
-  else dense_row<T, NPL, KEYS, WAVES, false>(a, one, row, 0);
-}
-
-template <typename T, int NPL, int KEYS, int WAVES, bool INDEXED>
-__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(const DenseArgs a,
-                                                                      const DenseSplit sp) {
-  dense_row<T, NPL, KEYS, WAVES, INDEXED>(a, sp, blockIdx.x, gridDim.x);
+template <typename T, int NPL, int KEYS, int WAVES, int INDEX>
+__global__ __launch_bounds__(64 * WAVES) void dense_attention_kernel(
+    const std::conditional_t<INDEX == 0, iak_dense_attention_args, DenseArgs> a, const DenseSplit sp) {
+  dense_row<T, NPL, KEYS, WAVES, INDEX>(a, sp, blockIdx.x, gridDim.x);
 }
 
 #include "dense_matrix.h"
@@ -350,11 +343,13 @@ __device__ __forceinline__ float block_reduce(float v, float* red) {
 // (splits <= MAX_SPLITS). The split weights go to the LDS; each context dim is
 // then summed over the splits by G thread groups (G = 256 / dims rounded up to
 // 64), each over every G-th split, with eight independent loads in flight.
-// FLAGS: the partials come from dense_matrix_kernel; a row of a batch entry with a
-// flagged key tile is computed again from its inputs.
+// accoff: where the contexts lie in ws; log2: the maxima are in the exp2 domain.
+// FLAGS: the partials come from dense_matrix_kernel with key-tile flags; a row of a
+// flagged batch entry is computed again from its inputs.
 template <typename T, bool FLAGS>
 __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseArgs a,
-                                                                    const DenseSplit sp, const MatrixPlan mp) {
+                                                                    const DenseSplit sp, const MatrixPlan mp,
+                                                                    int64_t accoff, int log2) {
   __shared__ float wt[MAX_SPLITS];
   __shared__ float red[MERGE_THREADS / 64];
   __shared__ float part[MERGE_THREADS];
@@ -363,7 +358,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
   const int i = (int)(row - b * a.q_len);
   if constexpr (FLAGS) {
     if (mx_flagged(mp, b)) {
-      dense_row_any<T, MX_MAX_DIM / 64, 2, MERGE_THREADS / 64>(a, row);
+      dense_row<T, MX_MAX_DIM / 64, 2, MERGE_THREADS / 64, ANY_INDEX>(a, DenseSplit{1, a.kv_len, nullptr}, row, 0);
       return;
     }
   }
@@ -371,7 +366,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
   const int64_t n = (int64_t)gridDim.x * S;
   const float* wm = sp.ws + row * S;
   const float* wl = sp.ws + n + row * S;
-  const float* wacc = sp.ws + sp.accoff + row * S * a.v_dim;
+  const float* wacc = sp.ws + accoff + row * S * a.v_dim;
   const float NEG_INF = -__builtin_inff();
   float mx = NEG_INF;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) mx = fmaxf(mx, wm[s]);
@@ -379,7 +374,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
   float ls = 0.f;
   for (int s = threadIdx.x; s < S; s += MERGE_THREADS) {
     // 0 for a range that saw no mass
-    const float w = wm[s] == NEG_INF ? 0.f : (sp.log2 ? __builtin_amdgcn_exp2f(wm[s] - M) : expf(wm[s] - M));
+    const float w = wm[s] == NEG_INF ? 0.f : (log2 ? __builtin_amdgcn_exp2f(wm[s] - M) : expf(wm[s] - M));
     wt[s] = w;
     ls += w * wl[s];
   }
@@ -420,35 +415,35 @@ __global__ __launch_bounds__(MERGE_THREADS) void dense_merge_kernel(const DenseA
 
 // MAXW: the most waves per workgroup whose registers and LDS fit (16 waves of
 // a 1,024-thread workgroup get 128 VGPRs each)
-template <typename T, int NPL, int KEYS, int MAXW, bool INDEXED>
+template <typename T, int NPL, int KEYS, int MAXW, int INDEX>
 void launch_items(const DenseArgs& a, const DenseSplit& sp, int64_t items, hipStream_t stream) {
   // waves per workgroup: about 4,096 waves in the grid (16 per CU), between 4 and MAXW
   const int64_t want = (4096 + items - 1) / items;
   const dim3 grid((unsigned)items);
   if (MAXW >= 16 && want >= 16)
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, MAXW >= 16 ? 16 : 4, INDEXED>), grid, dim3(1024), 0,
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, MAXW >= 16 ? 16 : 4, INDEX>), grid, dim3(1024), 0,
                        stream, a, sp);
   else if (want >= 8)
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 8, INDEXED>), grid, dim3(512), 0, stream, a, sp);
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 8, INDEX>), grid, dim3(512), 0, stream, a, sp);
   else
-    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 4, INDEXED>), grid, dim3(256), 0, stream, a, sp);
+    hipLaunchKernelGGL((dense_attention_kernel<T, NPL, KEYS, 4, INDEX>), grid, dim3(256), 0, stream, a, sp);
 }
 
-template <typename T, bool INDEXED>
+template <typename T, int INDEX>
 void launch_rows(const DenseArgs& a, const DenseSplit& sp, hipStream_t stream) {
   const int64_t rows = (int64_t)a.batch * a.q_len;
   const int64_t items = rows * sp.splits;
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
   const int npl = (width + 63) / 64;
   // keys per step: 2 * KEYS * NPL registers of K and V in flight per lane
-  if (npl <= 1) launch_items<T, 1, 8, 16, INDEXED>(a, sp, items, stream);
-  else if (npl <= 2) launch_items<T, 2, 8, 16, INDEXED>(a, sp, items, stream);
-  else if (npl <= 4) launch_items<T, 4, 4, 16, INDEXED>(a, sp, items, stream);
-  else if (npl <= 8) launch_items<T, 8, 4, 8, INDEXED>(a, sp, items, stream);
-  else launch_items<T, 16, 2, 8, INDEXED>(a, sp, items, stream);
+  if (npl <= 1) launch_items<T, 1, 8, 16, INDEX>(a, sp, items, stream);
+  else if (npl <= 2) launch_items<T, 2, 8, 16, INDEX>(a, sp, items, stream);
+  else if (npl <= 4) launch_items<T, 4, 4, 16, INDEX>(a, sp, items, stream);
+  else if (npl <= 8) launch_items<T, 8, 4, 8, INDEX>(a, sp, items, stream);
+  else launch_items<T, 16, 2, 8, INDEX>(a, sp, items, stream);
   if (sp.splits > 1)
     hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp,
-                       MatrixPlan{});
+                       MatrixPlan{}, 2 * items, 0);
 }
 
 // Splits per row: rows with SPLIT_MIN_KEYS keys or more on a short grid (fewer
@@ -456,7 +451,7 @@ void launch_rows(const DenseArgs& a, const DenseSplit& sp, hipStream_t stream) {
 // least RANGE_MIN_KEYS keys
 // (at most MAX_SPLITS ranges).
 DenseSplit split_plan(const DenseArgs& a) {
-  DenseSplit sp{1, a.kv_len, nullptr, 0, 0};
+  DenseSplit sp{1, a.kv_len, nullptr};
   const int64_t rows = (int64_t)a.batch * a.q_len;
   if (rows <= 0 || rows >= 512 || a.kv_len < SPLIT_MIN_KEYS) return sp;
   int64_t s = (SPLIT_TARGET_WGS + rows - 1) / rows;
@@ -467,7 +462,6 @@ DenseSplit split_plan(const DenseArgs& a) {
   const int64_t chunk = ((int64_t)a.kv_len + s - 1) / s;
   sp.splits = (int)(((int64_t)a.kv_len + chunk - 1) / chunk);
   sp.chunk = (int)chunk;
-  sp.accoff = 2 * rows * sp.splits;
   return sp;
 }
 
@@ -487,6 +481,17 @@ DenseSplit split_plan(const DenseArgs& a) {
 #define MX_MIN_ROWS_F32 3
 #endif
 
+// The float32 matrix instructions run at the rate of the row form's arithmetic, on 32
+// query rows at a time: where the keys are split (two launches) or the workgroups come
+// in two turns, the row form keeps calls of up to this many pairs if it takes one launch
+// itself (us per call among others, and waited for, row form / this one: 16 x 16 rows x 400 keys x 128 = 102,400
+// 19.7 / 24.1 and 42.8 / 43.9, 16 x 32 x 256 x 64 = 131,072 19.4 / 23.5 and 40.6 / 39.3, 300 x
+// 3 x 128 x 128 = 115,200 25.4 / 30.0; 16 x 32 x 400 x 64 = 204,800 22.2 / 24.1 and 46.8 / 39.7,
+// 100 x 16 x 256 x 64 38.5 / 23.6).
+#ifndef MX_TWO_TURN_PAIRS_F32
+#define MX_TWO_TURN_PAIRS_F32 131072
+#endif
+
 // 128 query rows by four waves over 64 keys, or by eight over 128: a step of one wave per
 // SIMD takes 3 us, of two (two workgroups on a CU, or the eight waves of one) 2.2 us for
 // each 64 keys, the one's matrix work under the other's softmax. Up to one workgroup per
@@ -500,29 +505,14 @@ DenseSplit split_plan(const DenseArgs& a) {
 #define MX_WIDE_WGS_CAUSAL 512
 #endif
 
+// scores that go through masks or positions
+bool general(const DenseArgs& a) { return a.mask || a.causal == IAK_CAUSAL_POSITIONS; }
+
 struct MatrixShape {
   int dp;       // dims, padded
   int qw, kw;   // waves over query rows and over keys
   int bkw;      // keys per wave and tile
 };
-
-// 16-byte pieces of whole elements on every operand, at most 256 dims
-bool matrix_applies(const DenseArgs& a) {
-  const int es = a.dtype == IAK_DTYPE_F32 ? 4 : 2, vec = 16 / es;
-  const double pairs = (double)a.batch * a.q_len * a.kv_len;
-  if (a.q_len < (es == 4 ? MX_MIN_ROWS_F32 : MX_MIN_ROWS) || pairs < (es == 4 ? MX_MIN_PAIRS_F32 : MX_MIN_PAIRS)) return false;
-  const int most = es == 4 ? MX_MAX_DIM_F32 : MX_MAX_DIM;
-  if (a.head_dim > most || a.v_dim > most || a.head_dim % vec || a.v_dim % vec) return false;
-  if (!(a.sm_scale > 0.f) || !std::isfinite(a.sm_scale)) return false;
-  const uintptr_t at = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
-                       reinterpret_cast<uintptr_t>(a.v);
-  if ((at & 15u) || (reinterpret_cast<uintptr_t>(a.out) & (4 * es - 1))) return false;
-  const int64_t row_strides = a.q_stride_t | a.k_stride_t | a.v_stride_t;
-  const int64_t batch_strides = a.batch > 1 ? (a.q_stride_b | a.k_stride_b | a.v_stride_b) : 0;
-  if ((row_strides | batch_strides) & (vec - 1)) return false;
-  if ((a.out_stride_t | (a.batch > 1 ? a.out_stride_b : 0)) & 3) return false;
-  return true;
-}
 
 // causal tiles past the diagonal are not visited
 bool causal_skip(const DenseArgs& a) { return a.causal == IAK_CAUSAL_TRIU && !a.mask && a.sm_scale <= 1.f; }
@@ -541,6 +531,49 @@ MatrixShape matrix_shape(const DenseArgs& a) {
   return s;
 }
 
+// Keys of a wave times dims up to which the keys are not split: the merge is a second
+// launch, 5 us of a short call, and costs more than it saves. us per call among others, and
+// waited for, all keys in one workgroup / split, float16: 16 x 16 rows x 400 keys x 128 =
+// 16,384 19.3 / 24.0 and 40.8 / 39.3, 16 x 16 x 1,000 x 64 = 16,384 19.0 / 23.9 and 41.3 /
+// 38.0, 8 x 64 x 600 x 64 = 20,480 19.3 / 24.2 and 43.0 / 39.1, 4 x 128 x 400 x 128 = 32,768
+// 23.0 / 24.1 and 47.3 / 43.2 (the row form 22 to 31 and 47 to 55); float32: 16 x 32 x 256 x
+// 64 = 4,096 19.0 / 23.7, x 400 = 8,192 22.2 / 23.7; float16 with a mask: 16 x 16 x 333 x
+// 80 = 9,216 31.9 / 36.5, 32 x 2 x 1,024 x 64 = 16,384 38 to 44 / 36.5.
+#ifndef MX_SHORT
+#define MX_SHORT 16384
+#define MX_SHORT_MASK 12288
+#define MX_SHORT_F32 6144
+#endif
+bool matrix_short(const DenseArgs& a, const MatrixShape& s) {
+  const int64_t bk = s.kw * s.bkw;
+  return s.dp <= 128 && ((int64_t)a.kv_len + bk - 1) / bk * s.bkw * s.dp <=
+         (a.dtype == IAK_DTYPE_F32 ? MX_SHORT_F32 : general(a) ? MX_SHORT_MASK : MX_SHORT);
+}
+
+// 16-byte pieces of whole elements on every operand, at most 256 dims
+bool matrix_applies(const DenseArgs& a) {
+  const int es = a.dtype == IAK_DTYPE_F32 ? 4 : 2, vec = 16 / es;
+  const double pairs = (double)a.batch * a.q_len * a.kv_len;
+  if (a.q_len < (es == 4 ? MX_MIN_ROWS_F32 : MX_MIN_ROWS) || pairs < (es == 4 ? MX_MIN_PAIRS_F32 : MX_MIN_PAIRS)) return false;
+  const int most = es == 4 ? MX_MAX_DIM_F32 : MX_MAX_DIM;
+  if (a.head_dim > most || a.v_dim > most || a.head_dim % vec || a.v_dim % vec) return false;
+  if (!(a.sm_scale > 0.f) || !std::isfinite(a.sm_scale)) return false;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k) |
+                       reinterpret_cast<uintptr_t>(a.v);
+  if ((at & 15u) || (reinterpret_cast<uintptr_t>(a.out) & (4 * es - 1))) return false;
+  const int64_t row_strides = a.q_stride_t | a.k_stride_t | a.v_stride_t;
+  const int64_t batch_strides = a.batch > 1 ? (a.q_stride_b | a.k_stride_b | a.v_stride_b) : 0;
+  if ((row_strides | batch_strides) & (vec - 1)) return false;
+  if ((a.out_stride_t | (a.batch > 1 ? a.out_stride_b : 0)) & 3) return false;
+  if (es == 4 && pairs <= MX_TWO_TURN_PAIRS_F32 && split_plan(a).splits == 1) {
+    const MatrixShape s = matrix_shape(a);
+    const int64_t wgs = (int64_t)a.batch * ((a.q_len + 32 * s.qw - 1) / (32 * s.qw));
+    const bool one_turn = wgs <= (s.dp > 64 ? 256 : 512);
+    if (!matrix_short(a, s) || !one_turn) return false;
+  }
+  return true;
+}
+
 // query tiles of 32 * qw rows; on short grids the keys go over about 256
 // workgroups in ranges of whole tiles
 MatrixPlan matrix_plan(const DenseArgs& a, const MatrixShape& s) {
@@ -549,16 +582,25 @@ MatrixPlan matrix_plan(const DenseArgs& a, const MatrixShape& s) {
   mp.nq = (int)((a.q_len + bq - 1) / bq);
   mp.nt = (int)((a.kv_len + bk - 1) / bk);
   mp.waves = s.qw * s.kw;
-  mp.skip = causal_skip(a);
   const int64_t wgs = (int64_t)a.batch * mp.nq;
   int64_t n = wgs > 0 && wgs < SPLIT_TARGET_WGS ? SPLIT_TARGET_WGS / wgs : 1;
+  const bool is_short = matrix_short(a, s);
+  if (is_short) n = 1;
   if (n > mp.nt) n = mp.nt;
   if (n > MAX_SPLITS) n = MAX_SPLITS;
   const int64_t per = ((int64_t)mp.nt + n - 1) / n;   // tiles per range
   mp.splits = (int)((mp.nt + per - 1) / per);
   mp.chunk = mp.splits > 1 ? (int)(per * bk) : a.kv_len;
   mp.accoff = (2 * (int64_t)a.batch * a.q_len * mp.splits + 3) / 4 * 4;
+  mp.again = is_short && a.dtype != IAK_DTYPE_F32;
+  mp.skip = !is_short && causal_skip(a);
   return mp;
+}
+
+// key-tile flags are needed where tiles are skipped, or a weight is split and not looked after
+// in the kernel
+bool matrix_flags(const DenseArgs& a, const MatrixPlan& mp) {
+  return mp.skip || (a.dtype != IAK_DTYPE_F32 && !mp.again);
 }
 
 size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
@@ -568,18 +610,27 @@ size_t matrix_partial_bytes(const DenseArgs& a, const MatrixPlan& mp) {
 
 size_t matrix_workspace(const DenseArgs& a) {
   const MatrixPlan mp = matrix_plan(a, matrix_shape(a));
-  return matrix_partial_bytes(a, mp) + (size_t)a.batch * mp.nt * mp.waves * sizeof(int32_t);
+  const size_t flags = matrix_flags(a, mp) ? (size_t)a.batch * mp.nt * mp.waves * sizeof(int32_t) : 0;
+  const size_t total = matrix_partial_bytes(a, mp) + flags;
+  return total ? total : IAK_DENSE_NO_SCRATCH;   // a workspace at all says that the form may run
+}
+
+template <typename T, int DP, int QW, int KW, int BKW, bool GEN>
+void launch_matrix_gen(const DenseArgs& a, const MatrixPlan& mp, hipStream_t stream) {
+  const dim3 grid((unsigned)((int64_t)a.batch * mp.nq * mp.splits)), block(64 * QW * KW);
+  if constexpr (sizeof(T) == 2 && DP <= 128) {
+    if (mp.again) {
+      hipLaunchKernelGGL((dense_short_kernel<T, DP, QW, KW, BKW, GEN>), grid, block, 0, stream, a, mp);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, GEN>), grid, block, 0, stream, a, mp);
 }
 
 template <typename T, int DP, int QW, int KW, int BKW>
 void launch_matrix_cfg(const DenseArgs& a, const MatrixPlan& mp, hipStream_t stream) {
-  const dim3 grid((unsigned)((int64_t)a.batch * mp.nq * mp.splits));
-  if (a.mask || a.causal == IAK_CAUSAL_POSITIONS)
-    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, true>), grid, dim3(64 * QW * KW), 0, stream,
-                       a, mp);
-  else
-    hipLaunchKernelGGL((dense_matrix_kernel<T, DP, QW, KW, BKW, false>), grid, dim3(64 * QW * KW), 0, stream,
-                       a, mp);
+  if (general(a)) launch_matrix_gen<T, DP, QW, KW, BKW, true>(a, mp, stream);
+  else launch_matrix_gen<T, DP, QW, KW, BKW, false>(a, mp, stream);
 }
 
 template <typename T, int DP>
@@ -601,7 +652,8 @@ void launch_matrix(const DenseArgs& a, void* workspace, hipStream_t stream) {
   const MatrixShape s = matrix_shape(a);
   MatrixPlan mp = matrix_plan(a, s);
   mp.ws = static_cast<float*>(workspace);
-  mp.flags = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + matrix_partial_bytes(a, mp));
+  const bool flags = matrix_flags(a, mp);
+  if (flags) mp.flags = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) + matrix_partial_bytes(a, mp));
   if (s.dp == 64) launch_matrix_dims<T, 64>(a, s, mp, stream);
   else if (s.dp == 128) launch_matrix_dims<T, 128>(a, s, mp, stream);
   if constexpr (sizeof(T) == 2) {
@@ -611,10 +663,15 @@ void launch_matrix(const DenseArgs& a, void* workspace, hipStream_t stream) {
   }
   const int64_t rows = (int64_t)a.batch * a.q_len;
   if (mp.splits > 1) {
-    const bool gen = a.mask || a.causal == IAK_CAUSAL_POSITIONS;
-    const DenseSplit sp{mp.splits, mp.chunk, mp.ws, mp.accoff, gen ? 0 : 1};
-    hipLaunchKernelGGL((dense_merge_kernel<T, true>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp);
-  } else {
+    const DenseSplit sp{mp.splits, mp.chunk, mp.ws};
+    const int log2 = general(a) ? 0 : 1;
+    if (flags)
+      hipLaunchKernelGGL((dense_merge_kernel<T, true>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp,
+                         mp.accoff, log2);
+    else
+      hipLaunchKernelGGL((dense_merge_kernel<T, false>), dim3((unsigned)rows), dim3(MERGE_THREADS), 0, stream, a, sp, mp,
+                         mp.accoff, log2);
+  } else if (flags) {
     const int64_t per = a.batch < 256 ? (256 + a.batch - 1) / a.batch : 1;
     hipLaunchKernelGGL(dense_fixup_kernel<T>, dim3((unsigned)(a.batch * per)), dim3(256), 0, stream, a, mp);
   }
@@ -624,29 +681,47 @@ template <typename T>
 void launch_typed(const DenseArgs& a, void* workspace, hipStream_t stream) {
   if (workspace && matrix_applies(a)) return launch_matrix<T>(a, workspace, stream);
   DenseSplit sp = split_plan(a);
-  if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr, 0, 0};
+  if (!workspace) sp = DenseSplit{1, a.kv_len, nullptr};
   sp.ws = static_cast<float*>(workspace);
-  if (a.kv_index) launch_rows<T, true>(a, sp, stream);
-  else launch_rows<T, false>(a, sp, stream);
+  if (a.kv_index) launch_rows<T, 1>(a, sp, stream);
+  else launch_rows<T, 0>(a, sp, stream);
 }
 
 }  // namespace
 
+// One object per element type (the Makefile compiles this file three times, side by side).
+#if defined(IAK_DENSE_F16)
+hipError_t launch_dense_f16(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
+                            hipStream_t stream) {
+  launch_typed<_Float16>(DenseArgs{args, kv_index}, workspace, stream);
+  return hipGetLastError();
+}
+#elif defined(IAK_DENSE_BF16)
+hipError_t launch_dense_bf16(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
+                             hipStream_t stream) {
+  launch_typed<bf16_bits>(DenseArgs{args, kv_index}, workspace, stream);
+  return hipGetLastError();
+}
+#else
+hipError_t launch_dense_f16(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
+                            hipStream_t stream);
+hipError_t launch_dense_bf16(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
+                             hipStream_t stream);
+
 size_t dense_attention_workspace(const iak_dense_attention_args& args) {
   const DenseArgs a{args, nullptr};   // the keys' rows change no size
+  if (matrix_applies(a)) return matrix_workspace(a);
   const DenseSplit sp = split_plan(a);
-  const size_t rows = sp.splits <= 1 ? 0 : (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.v_dim) * sizeof(float);
-  const size_t matrix = matrix_applies(a) ? matrix_workspace(a) : 0;
-  return rows > matrix ? rows : matrix;
+  return sp.splits <= 1 ? 0 : (size_t)a.batch * a.q_len * sp.splits * (2 + (size_t)a.v_dim) * sizeof(float);
 }
 
 hipError_t launch_dense_attention(const iak_dense_attention_args& args, const int64_t* kv_index, void* workspace,
                                   hipStream_t stream) {
-  const DenseArgs a{args, kv_index};
-  if (a.dtype == IAK_DTYPE_F32) launch_typed<float>(a, workspace, stream);
-  else if (a.dtype == IAK_DTYPE_F16) launch_typed<_Float16>(a, workspace, stream);
-  else launch_typed<bf16_bits>(a, workspace, stream);
+  if (args.dtype == IAK_DTYPE_F16) return launch_dense_f16(args, kv_index, workspace, stream);
+  if (args.dtype == IAK_DTYPE_BF16) return launch_dense_bf16(args, kv_index, workspace, stream);
+  launch_typed<float>(DenseArgs{args, kv_index}, workspace, stream);
   return hipGetLastError();
 }
+#endif
 
 }  // namespace iak

@@ -21,6 +21,7 @@ IAK_OK, IAK_EINVAL, IAK_ENOTSUP, IAK_EHIP = 0, 1, 2, 3
 TAG_FP16, TAG_INT8, TAG_SKIP, TAG_FP8, TAG_INT4, TAG_INT4_RESIDUAL = 0, 1, 2, 3, 4, 5
 DTYPE_F16, DTYPE_F32, DTYPE_BF16 = 0, 1, 2
 MASK_BOOL = 3
+DENSE_NO_SCRATCH = 16   # IAK_DENSE_NO_SCRATCH
 CAUSAL_NONE, CAUSAL_TRIU, CAUSAL_POSITIONS = 0, 1, 2
 
 c_i32, c_i64, c_void_p, c_float = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p, ctypes.c_float

@@ -146,7 +146,11 @@ def _dense_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, causal: 
     # above and the workspace were allocated on this stream, so the caching
     # allocator reuses their memory only after these kernels
     ws_bytes = N.dense_attention_workspace(a)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
+    ws = None
+    if ws_bytes > N.DENSE_NO_SCRATCH:
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+    elif ws_bytes:
+        ws = out                              # nothing is written to it as a workspace
     N.dense_attention(a, current_stream_handle(dev), ws.data_ptr() if ws is not None else 0, ws_bytes,
                       kv_index.data_ptr() if kv_index is not None else 0)
     return out

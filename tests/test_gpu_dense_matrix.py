@@ -178,19 +178,22 @@ def test_waves_per_workgroup(heads, t, tk, d, dt, monkeypatch):
 
 
 # key counts one short of a 32- or 128-key tile, one past it, and whole tiles; the wave shapes of
-# few, some and many query rows, keys split over workgroups (2 and 8 heads) and not (300)
+# few, some and many query rows, keys split over workgroups (2 to 8 heads) and not, short calls
+# (up to 256 keys of a wave x 64 dims) and long ones
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
-@pytest.mark.parametrize("heads,tq,tk", [(8, 8, 1055), (2, 40, 1025), (2, 128, 1057), (300, 8, 159), (300, 8, 161),
-                                         (300, 33, 65), (300, 130, 33)])
-def test_special_values_in_the_last_key(heads, tq, tk, dt, monkeypatch):
+@pytest.mark.parametrize("heads,tq,tk,d", [(8, 8, 1055, 64), (2, 40, 1025, 64), (2, 128, 1057, 64), (300, 8, 159, 64),
+                                           (300, 8, 161, 64), (300, 33, 65, 64), (300, 130, 33, 64), (2, 128, 257, 64),
+                                           (64, 20, 129, 128), (40, 60, 95, 96), (130, 150, 128, 128),
+                                           (260, 130, 400, 128)])
+def test_special_values_in_the_last_key(heads, tq, tk, d, dt, monkeypatch):
     """The last key's row stands in for the keys that fill up its tile: whatever it holds, the
     result is the row form's. Its score is up to 2^7 above the others', as far as the
     running maximum may lag, so a large finite value must not overflow on the way either."""
     from intent_attention import BlockLayout, BlockPolicy, SemanticBlock, dense_attention, semantic_block_attention
-    q, k, v, g = _qkv(heads + tk, (heads,), tq, tk, 64, 64, dt)
+    q, k, v, g = _qkv(heads + tk, (heads,), tq, tk, d, d, dt)
     q[..., 0], k[:, :-1] = 4.0, k[:, :-1] * 0.1
     k[:, -1] = 0.0
-    k[:, -1, 0] = 9.0                                  # 4 * 9 / 8 log2(e) = 6.5
+    k[:, -1, 0] = 9.0 / 8 * d ** 0.5                   # 4 * 9 / 8 log2(e) = 6.5
     big = 60000.0 if dt == "f16" else 1e37
     mask = torch.zeros(tq, tk).to(DT[dt])
     mask[:, 5] = float("-inf")
