@@ -14,15 +14,16 @@
 //           lane: keys 8 (r / 4) + 4 h + r % 4.
 //   softmax per lane over its keys, one lane swap with lane ^ 32 for the other
 //           half; the running max moves only when a tile exceeds it by more
-//           than 2^8, so the accumulators are rarely rescaled.
+//           than 2^8 (float16 2^3, float32 at once), so the accumulators are rarely
+//           rescaled.
 //   values  O^T[32 dims x 32 rows] += V^T . P^T: P is the score result as it
 //           lies in the registers, V^T comes out of the [key][dim] tile
 //           (16-bit: the transposing read ds_read_b64_tr_b16).
 // Arithmetic. Every product is exact or float32 and every sum is float32.
 // float16 / bfloat16 inputs: Q.K products are exact on the 16-bit matrix
 // instructions; the float32 weights are split into 16-bit parts whose sum
-// carries 22 bits or more (float16: two parts of p * 2^7, bfloat16: three),
-// one matrix instruction per part. float32 inputs: v_mfma_f32_32x32x2_f32.
+// carries 22 bits or more (float16: two parts of p * 2^12, to 2^-37 of the row's
+// largest weight; bfloat16: three), one matrix instruction per part. float32 inputs: v_mfma_f32_32x32x2_f32.
 //
 // Non-finite and large values come out as in the plain sum. Four shortcuts would answer
 // differently for them: a split weight times an infinite V (inf * 0 in the low part);
@@ -32,11 +33,10 @@
 // overflowing score there makes its row NaN, an infinite V a zero weight's
 // product NaN).
 //   float32 rows, and 16-bit ones of short calls (dense_short_kernel): V of the keys past
-//           the range is zeros, and the maximum does not lag (a float16 V cannot
-//           overflow: there it may). A workgroup of a short call whose rows end in a sum
-//           that is not finite walks its keys once more, with 1 for every weight above 0:
-//           the sums are infinite or NaN where the plain ones are, and those are
-//           written.
+//           the range is zeros, and the maximum does not lag (float16: by 2^3, its V cannot
+//           overflow). A workgroup of a short call whose rows end in a sum that is not
+//           finite walks its keys once more, with 1 for every weight above 0: the sums
+//           are infinite or NaN where the plain ones are, and those are written.
 //   the others, and every call with tiles that are not visited: each key tile is checked
 //           once, by one of the workgroups that loads it, and its flag (K and V below
 //           2^59 or not) goes to the workspace; the kernel that follows (the merge,
@@ -54,9 +54,6 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 constexpr int MX_MAX_DIM = 256;      // 16-bit inputs
 constexpr int MX_MAX_DIM_F32 = 128;  // float32: Q, scores and context of wider rows spill
 constexpr float LOG2E = 1.44269504088896340736f;
-// float16 weights are kept as p * 2^MX_P_EXP (<= 2^15): the low part's
-// subnormal step is then 2^-31 of the row's largest weight
-constexpr float MX_P_EXP = 7.0f;
 constexpr float LARGE = 1e5f;   // scores (exp2 domain) whose rounding reaches 2^-8
 
 struct MatrixPlan {

@@ -212,3 +212,28 @@ def test_special_values_in_the_last_key(heads, tq, tk, d, dt, monkeypatch):
             live = torch.isfinite(want)
             scale = want[live].double().abs().clamp(min=1)
             assert float(((got[live].double() - want[live].double()) / scale).abs().max()) <= 2 * TOL[dt], what
+
+
+@pytest.mark.parametrize("mask", [False, True])
+@pytest.mark.parametrize("tq,tk", [(32, 700), (64, 300), (200, 130)])
+def test_small_float16_weights(tq, tk, mask):
+    """Keys whose weights are 2^-14 to 2^-30 of the largest, with values that make up for it: the
+    weights keep what they had in float32 down to 2^-37 of the largest one (half the smallest
+    float16 step after the 2^12 they are kept at), the output its own rounding of 2^-11."""
+    from intent_attention import dense_attention
+    g = torch.Generator().manual_seed(tq)
+    q = torch.zeros(1, 2, tq, 64)
+    q[..., 0] = torch.linspace(10, 21, tq).half().float()
+    k, v = torch.randn(1, 2, tk, 64, generator=g) * 0.3, 30000 + 30000 * torch.rand(1, 2, tk, 64, generator=g)
+    k[..., 0], k[:, :, 40, 0] = torch.rand(1, 2, tk, generator=g) * 0.2, 8.0
+    v[:, :, 40] = 0.0
+    q, k, v = q.half(), k.half(), v.half()
+    m = torch.zeros(tq, tk).half() if mask else None
+    got = dense_attention(q.cuda(), k.cuda(), v.cuda(), mask=None if m is None else m.cuda()).double().cpu()
+    p = torch.softmax(q.double() @ k.double().transpose(-1, -2) / 8, -1)
+    want = p @ v.double()
+    # float32 sums besides (2e-5 as above), of the scores too: 21 * 2^-22
+    bound = want.abs() * (2 ** -11 + 4e-5) + 2 ** -37 * p.amax(-1, keepdim=True) * v.double().abs().sum(-2, keepdim=True)
+    worst = float(((got - want).abs() / bound).max())
+    print(f"[gpu-case] {tq}x{tk} mask={mask}: error / bound {worst:.2f}", flush=True)
+    assert worst <= 1.0
