@@ -240,7 +240,9 @@ __global__ __launch_bounds__(64 * WAVES, 1) void mla_rows_matrix_kernel(const ia
       mx = fmaxf(mx, s[r]);
     }
     mx = rx_max32(mx);
-    const bool grow = mx > m + RESCALE_SLACK;
+    // the maximum does not lag: a weight above 1 would take a large latent that the scores
+    // do not see (its query dim 0) over the range
+    const bool grow = mx > m;
     if (__builtin_amdgcn_ballot_w64(grow)) {
       const float alpha = grow ? __builtin_amdgcn_exp2f(m - mx) : 1.f;   // 0 at first (m = -inf)
       l *= alpha;

@@ -53,3 +53,24 @@ def test_nonfinite_latents_as_the_rows_form(value):
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
     live = torch.isfinite(want)
     assert float((got[live] - want[live]).abs().max()) <= 2e-5 * max(1.0, float(want[live].abs().max()))
+
+
+@pytest.mark.parametrize("dc", [128, 512, 768])
+@pytest.mark.parametrize("c_dt", ["float32", "bfloat16"])
+def test_large_latents_that_stay_finite(dc, c_dt):
+    """A latent of 1e37 that the scores do not see (its query dim is zero), in a key that scores 2^6
+    above the tile before it: its weight must not pass 1 on the way to a context that is finite."""
+    from intent_attention.triton_mla_decode import mla_latent_context
+    g = torch.Generator().manual_seed(dc)
+    n = 9216 if dc == 768 else 1152            # with and without the keys split over workgroups
+    B = 40 if dc == 768 else 9000
+    q, C = torch.randn(B, 1, dc, generator=g), torch.randn(n, dc, generator=g) * 0.1
+    q[..., 0], q[..., 5] = 8.0, 0.0
+    C[35] = 0.0
+    C[35, 0], C[35, 5] = 4.3 * dc ** 0.5 / 8, 1e37       # exp(4.3) = 2^6.2
+    q, C = q.cuda(), C.to(getattr(torch, c_dt)).cuda()
+    ids = torch.arange(n // 64, dtype=torch.int32).cuda()
+    got = mla_latent_context(q, C, ids, 64)
+    want = _ref(q, C, ids, 64)
+    assert bool(got.isfinite().all())
+    assert float(((got.double() - want).abs() / want.abs().clamp(min=1)).max()) <= 2e-5
