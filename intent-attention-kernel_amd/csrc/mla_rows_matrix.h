@@ -87,7 +87,7 @@ __global__ __launch_bounds__(64 * WAVES, 1) void mla_rows_matrix_kernel(const ia
   constexpr int PPK = DW / EPC;                     // pieces of a key in the wave's part
   constexpr int NCH = RX_KEYS * PPK / 64;           // pieces per lane and tile
   static_assert(RX_KEYS * PPK % 64 == 0, "whole pieces per lane");
-  __shared__ char tile_lds[WAVES][RX_KEYS * RB];
+  __shared__ __attribute__((aligned(16))) char tile_lds[WAVES][RX_KEYS * RB];   // read in 16-byte pieces
   __shared__ float part_s[WAVES][16][64];
   const int nw = blockDim.x >> 6;
   const int lane = threadIdx.x & 63;
