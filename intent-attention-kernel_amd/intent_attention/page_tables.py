@@ -78,7 +78,7 @@ def _upload(arrays, dev: torch.device) -> List[torch.Tensor]:
         total += max(a.size, 1)              # a valid pointer for an empty array
     if host:
         pinned = uploads_pinned(dev)
-        staged = torch.empty(total, dtype=torch.int32, pin_memory=pinned)
+        staged = torch.empty(total, dtype=torch.int32, device="cpu", pin_memory=pinned)   # whatever torch's default device
         view = staged.numpy()
         for _, at, a in host:
             view[at:at + max(a.size, 1)] = a if a.size else 0
