@@ -36,6 +36,7 @@ no score first (``_resolve_dynamic_scores`` :52-78 with the cosine probe of
 from __future__ import annotations
 
 import math
+from operator import index
 from typing import Any, Dict, List, Optional, Tuple, Union
 
 import numpy as np
@@ -201,7 +202,7 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     kv_tokens = k.size(-2)
     dynamic = _resolve_dynamic_scores(q, k, layout)
     layout.validate(kv_tokens)
-    spans = [(b.start, b.end) for b in layout.selected_blocks()]
+    spans = [(index(b.start), index(b.end)) for b in layout.selected_blocks()]   # whole numbers, as range takes them
     if not spans:
         out = torch.zeros_like(q)
         if not return_debug:
