@@ -202,8 +202,13 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     kv_tokens = k.size(-2)
     dynamic = _resolve_dynamic_scores(q, k, layout)
     layout.validate(kv_tokens)
-    spans = [(index(b.start), index(b.end)) for b in layout.selected_blocks()]   # whole numbers, as range takes them
-    if not spans:
+    own = getattr(layout.selected_token_indices, "__func__", None) is not BlockLayout.selected_token_indices
+    if own:                                   # a layout that selects its tokens itself
+        spans, tokens = [], layout.selected_token_indices()
+    else:
+        spans = [(index(b.start), index(b.end)) for b in layout.selected_blocks()]   # whole numbers, as range takes them
+        tokens = any(e > s for s, e in spans)
+    if not tokens:
         out = torch.zeros_like(q)
         if not return_debug:
             return out
@@ -212,8 +217,9 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         if dynamic:
             debug["dynamic_scores"] = dynamic
         return out, debug
-    idx = _token_index(spans, k.device)
-    if _index_in_place(q, k, v):
+    idx = torch.tensor(tokens, dtype=torch.long, device=k.device) if own else _token_index(spans, k.device)
+    # (the kernel reads rows as they are named: only tokens that are known to be inside)
+    if not own and all(0 <= s <= e <= kv_tokens for s, e in spans) and _index_in_place(q, k, v):
         out = _dense_attention(q, k, v, causal, None, idx, kv_index=idx)
     else:
         out = dense_attention(q, k.index_select(-2, idx), v.index_select(-2, idx), causal=causal,

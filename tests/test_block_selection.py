@@ -46,3 +46,32 @@ def test_bounds_that_are_not_whole_numbers_are_refused(calls, bounds):
     with pytest.raises(TypeError, match="integer"):
         reference.semantic_block_attention(*_qkv(), _layout(BlockLayout, bounds))
     assert not calls
+
+
+class _EveryThird(BlockLayout):
+    def selected_token_indices(self):
+        return super().selected_token_indices()[::3]
+
+
+class _Outside(BlockLayout):
+    def validate(self, total_tokens):
+        pass
+
+
+def test_a_layout_that_selects_its_own_tokens(calls):
+    reference.semantic_block_attention(*_qkv(), _layout(_EveryThird, (0, 3), (7, 12)))
+    one = _layout(BlockLayout, (0, 30))
+    one.selected_token_indices = lambda: [4, 2, 2]
+    _, debug = reference.semantic_block_attention(*_qkv(), one, return_debug=True)
+    assert calls == [("gathered", [0, 7, 10]), ("gathered", [4, 2, 2])] and debug["selected_kv_tokens"] == 3
+    one.selected_token_indices = lambda: []
+    out = reference.semantic_block_attention(*_qkv(), one)
+    assert len(calls) == 2 and not out.any()
+
+
+@pytest.mark.parametrize("bounds", [(30, 50), (-2, 5)])
+def test_tokens_outside_are_not_read_in_place(calls, bounds):
+    """Without BlockLayout's validation the gather is what checks the tokens (index_select raises)."""
+    with pytest.raises((IndexError, RuntimeError)):
+        reference.semantic_block_attention(*_qkv(), _layout(_Outside, bounds))
+    assert not calls
