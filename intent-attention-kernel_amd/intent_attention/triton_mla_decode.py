@@ -88,13 +88,14 @@ def _projects(ctx: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the projection runs on libiak's kernel, which reads W as it is stored: up to
     MAX_PROJECT_ROWS rows over whole 8 x 32 pieces of a row-major W. Wherever torch would do
     more than multiply (a W that is differentiated, in either mode, mapped over, sparse or a
-    subclass; autocast), and for more rows, torch's float32 GEMM over W.float() keeps it."""
+    subclass; autocast; a trace or a dispatch mode, which records the product), and for more rows, torch's float32 GEMM over W.float() keeps it."""
     return (type(w) in (torch.Tensor, torch.nn.Parameter) and w.layout is torch.strided and w.dtype in _DT
             and 0 < ctx.shape[0] * ctx.shape[1] <= MAX_PROJECT_ROWS
             and not w.is_neg() and w.stride(1) == 1 and w.shape[0] % 8 == 0 and w.shape[1] % 32 == 0 and w.shape[1] > 0
             and not (w.requires_grad and torch.is_grad_enabled()) and _fwd_ad._current_level < 0
             and not torch._C._functorch.is_functorch_wrapped_tensor(w)
-            and not torch.is_autocast_enabled(ctx.device.type))
+            and not torch.is_autocast_enabled(ctx.device.type)
+            and torch._C._get_tracing_state() is None and not torch._C._len_torch_dispatch_stack())
 
 
 def mla_decode_triton(q_absorb: torch.Tensor, C: torch.Tensor, W_VO_fused: torch.Tensor,
