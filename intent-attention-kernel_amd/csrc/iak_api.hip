@@ -226,19 +226,27 @@ iak_status validate(const iak_paged_decode_args* a, Plan* plan, bool tiers = tru
   return IAK_OK;
 }
 
-// The few-heads MLA form is taken for at most 16 heads, unless they read FP8 / INT8
+// The few-heads MLA form is taken for at most 16 heads, unless they read only FP8 / INT8
 // latents of 512 dims or more (which each wave then converts for itself), and for
 // more heads over one or two short tables, where its workgroups per 16 heads use
-// more of the chip. Both forms, us per call (split kernel and merge): 16 heads x
-// 576 dims, float16, 8 x 300 pages 28.5 / 25.1, 32 x 512 99.0 / 77.7; FP8 / INT8
-// 8 x 300 24.6 / 26.4; 8 heads 23.9 / 23.8; 16 heads x 128 dims 8 x 300 14.6 /
-// 12.2, 32 x 512 44.6 / 34.0; 1 x 512 pages, 64 heads x 576 34.7 / 24.1; 8 x 300,
-// 32 heads x 576 30.5 / 30.1, 64 heads 35.1 / 42.8.
+// more of the chip; over one-byte latents alone, up to 512 pages. Both forms, us per call
+// in a graph (split kernel and merge), 576 dims:
+//   16 heads, float16 8 x 301 pages 29.2 / 26.1, 32 x 512 106 / 80, 32 x 8 17.7 / 15.6; pools with
+//   float16 and one-byte pages, a third of them float16 30.5 / 28.4, 101 / 81, 18.1 / 17.0,
+//   none of them 28.8 / 29.5, 89 / 83, 18.2 / 17.0 (1 x 64 pages 15.6 / 16.8); one-byte pools
+//   8 x 300 24.6 / 26.4 (8 heads 23.9 / 23.8); 128 dims 8 x 300 14.6 / 12.2;
+//   64 heads, 1 x 512 pages 34.7 / 24.1, 2 x 512 (4,096 visits) 31.1 / 28.6; 128 heads 1 x 512 39.6 /
+//   28.7, 2 x 256 36.5 / 28.3; 32 heads 1 x 2,048 37.0 / 32.4, 2 x 1,024 32.1 / 30.1; 8 x 300, 32 heads
+//   30.5 / 30.1, 64 heads 35.1 / 42.8; one-byte pools 128 heads 1 x 512 38.9 / 31.2, 64 heads 2 x
+//   256 26.5 / 23.3, but 2 x 512 29.6 / 31.2, 48 heads 2 x 512 27.3 / 31.4, 32 heads 2 x 1,024
+//   29.8 / 33.3, 1 x 1,024 29.0 / 26.8.
 constexpr long long MLA_FEW_VISITS = 4096;   // pages x groups of 16 heads
+constexpr long long MLA_FEW_CODE_PAGES = 512;
 bool mla_few_heads(const iak_mla_decode_args* a, bool fp16) {
   if (a->num_heads <= 16 && (a->num_heads <= 8 || fp16 || a->qk_dim <= 256)) return true;
-  return a->num_heads > 16 && a->batch <= 2 &&
-         (long long)a->batch * a->table_width * ((a->num_heads + 15) / 16) <= MLA_FEW_VISITS;
+  const long long pages = (long long)a->batch * a->table_width;
+  return a->num_heads > 16 && a->batch <= 2 && pages * ((a->num_heads + 15) / 16) <= MLA_FEW_VISITS &&
+         (fp16 || pages <= MLA_FEW_CODE_PAGES);
 }
 
 struct MPlan {
