@@ -74,3 +74,26 @@ def test_large_latents_that_stay_finite(dc, c_dt):
     want = _ref(q, C, ids, 64)
     assert bool(got.isfinite().all())
     assert float(((got.double() - want).abs() / want.abs().clamp(min=1)).max()) <= 2e-5
+
+
+def test_without_a_workspace_few_rows_take_the_rows_form():
+    """A C caller may pass no workspace; the keys are not split then, and 32 rows go to the
+    rows form, as 15 do: each row bit for bit the same in both calls."""
+    from intent_attention import _native as N
+    from intent_attention.decode_core import current_stream_handle
+    g = torch.Generator().manual_seed(2)
+    q, C = torch.randn(32, 1, 576, generator=g).cuda(), torch.randn(8192, 576, generator=g).half().cuda()
+    ids = torch.arange(128, dtype=torch.int32).cuda()
+    out = []
+    for rows in (15, 32):
+        ctx = torch.empty(rows, 1, 576, device="cuda")
+        a = N.MlaRowsArgs()
+        a.batch, a.q_len, a.latent_dim, a.page_size, a.num_selected, a.num_rows = rows, 1, 576, 64, 128, 8192
+        a.q, a.q_dtype, a.q_stride_b, a.q_stride_t = q.data_ptr(), N.DTYPE_F32, 576, 576
+        a.latents, a.latent_dtype, a.latent_stride = C.data_ptr(), N.DTYPE_F16, 576
+        a.page_ids, a.context, a.sm_scale = ids.data_ptr(), ctx.data_ptr(), 1 / 24.0
+        N.mla_decode_rows(a, current_stream_handle(ctx.device))
+        out.append(ctx)
+    assert torch.equal(out[0], out[1][:15])
+    ref = _ref(q, C, ids, 64)
+    assert float((out[1].double() - ref).abs().max() / ref.abs().max()) <= 2e-5
