@@ -36,7 +36,6 @@ no score first (``_resolve_dynamic_scores`` :52-78 with the cosine probe of
 from __future__ import annotations
 
 import math
-from operator import index
 from typing import Any, Dict, List, Optional, Tuple, Union
 
 import numpy as np
@@ -177,9 +176,9 @@ def _resolve_dynamic_scores(q: torch.Tensor, k: torch.Tensor, layout: BlockLayou
     return dynamic
 
 
-def _token_index(spans: List[Tuple[int, int]], dev: torch.device) -> torch.Tensor:
+def _token_index(spans: List[range], dev: torch.device) -> torch.Tensor:
     """The token indices of the spans in order, int64 on the device."""
-    idx = torch.from_numpy(np.concatenate([np.arange(s, e, dtype=np.int64) for s, e in spans]))
+    idx = torch.from_numpy(np.concatenate([np.arange(r.start, r.stop, dtype=np.int64) for r in spans]))
     if not uploads_pinned(dev):
         return idx.to(dev)
     return idx.pin_memory().to(dev, non_blocking=True)
@@ -202,13 +201,12 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     kv_tokens = k.size(-2)
     dynamic = _resolve_dynamic_scores(q, k, layout)
     layout.validate(kv_tokens)
-    own = getattr(layout.selected_token_indices, "__func__", None) is not BlockLayout.selected_token_indices
-    if own:                                   # a layout that selects its tokens itself
-        spans, tokens = [], layout.selected_token_indices()
-    else:
-        spans = [(index(b.start), index(b.end)) for b in layout.selected_blocks()]   # whole numbers, as range takes them
-        tokens = any(e > s for s, e in spans)
-    if not tokens:
+    # a plain BlockLayout's blocks are inside the keys (validate) and are what it selects; a
+    # layout with methods of its own is asked for its tokens
+    plain = type(layout) is BlockLayout and len(vars(layout)) == 1
+    selected: Any = [range(b.start, b.end) for b in layout.selected_blocks()] if plain \
+        else layout.selected_token_indices()
+    if not selected:
         out = torch.zeros_like(q)
         if not return_debug:
             return out
@@ -217,9 +215,9 @@ def semantic_block_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         if dynamic:
             debug["dynamic_scores"] = dynamic
         return out, debug
-    idx = torch.tensor(tokens, dtype=torch.long, device=k.device) if own else _token_index(spans, k.device)
+    idx = _token_index(selected, k.device) if plain else torch.tensor(selected, dtype=torch.long, device=k.device)
     # (the kernel reads rows as they are named: only tokens that are known to be inside)
-    if not own and all(0 <= s <= e <= kv_tokens for s, e in spans) and _index_in_place(q, k, v):
+    if plain and _index_in_place(q, k, v):
         out = _dense_attention(q, k, v, causal, None, idx, kv_index=idx)
     else:
         out = dense_attention(q, k.index_select(-2, idx), v.index_select(-2, idx), causal=causal,
