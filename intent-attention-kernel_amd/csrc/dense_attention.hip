@@ -15,7 +15,7 @@
 //
 // Calls with several query rows per batch entry run on the matrix cores
 // (dense_matrix.h: causal prefill of 32 heads x 2,048 rows x 128 in float16
-// 10.8 ms -> 0.082 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 18 us);
+// 10.8 ms -> 0.082 ms, 128 rows x 3,072 keys x 64 in float32, 8 heads, 274 -> 21 us);
 // what follows is the rows form, for the rest.
 //
 // Selected tokens (kv_index) are read where they lie: the gathered K and V of 3,072 of
@@ -521,7 +521,7 @@ MatrixShape matrix_shape(const DenseArgs& a) {
   const int width = a.head_dim > a.v_dim ? a.head_dim : a.v_dim;
   MatrixShape s{64, 4, 1, 64};
   const bool f32 = a.dtype == IAK_DTYPE_F32;
-  s.dp = width <= 64 ? 64 : (width <= 96 && !f32) ? 96 : width <= 128 ? 128 : width <= 192 ? 192 : 256;
+  s.dp = width <= 64 ? 64 : (width <= 96 && !f32) ? 96 : width <= 128 || f32 ? 128 : width <= 192 ? 192 : 256;
   if (f32) s.bkw = 32;
   // few query rows: the four waves share out the keys instead
   if (a.q_len <= 32 && s.dp <= 128) s.qw = 1, s.kw = 4, s.bkw = 32;

@@ -7,8 +7,8 @@
 // the LDS, added pairwise. Every product is a float32 product and every sum float32.
 // Bound: the chain of launch, W's first line and the waves' meeting; W is 4.7 MB at
 // 576 x 4,096 in float16, 1 us at the rate of HBM. 32 rows x 576 x 4,096, us per call:
-// W to float32 and a library GEMM 24.7 to 35, this 7.0; 128 rows 24.7 / 11.0; 32 rows x 128 x
-// 1,024 23.1 / 3.8. Error against float64 4.3e-7 -> 1.6e-7 (the waves' short chains).
+// W to float32 and a library GEMM 24.7 to 35, this 7.0 (the kernel's trace, which includes its
+// start, 8.9); 128 rows 24.7 / 11.0; 32 rows x 128 x 1,024 23.1 / 3.8. Error against float64 4.3e-7 -> 1.6e-7 (the waves' short chains).
 #ifndef IAK_MLA_PROJECT_H
 #define IAK_MLA_PROJECT_H
 

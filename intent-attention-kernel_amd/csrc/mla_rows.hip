@@ -7,7 +7,7 @@
 // (p+1)*page_size - 1 of C [rows, d_c], the last page of C possibly shorter --
 // with scores (q . c) * sm_scale in float32, an online softmax, and context =
 // sum(p c) / sum(p); zeros when no row is visited. The projection by W_VO
-// that follows is a plain GEMM outside this file.
+// that follows is mla_project.h's kernel, or torch's GEMM (see there).
 //
 // This is the reference API's arithmetic, not the serving path: the MFMA
 // kernel of mla_decode.hip computes over paged f16 / FP8 / INT8 pools with f16
@@ -99,7 +99,7 @@ struct RowSplit {
   int chunk;         // keys per workgroup (the last may have fewer)
   int nkeys;         // num_selected * page_size
   uint32_t magic;    // floor(2^32 / page_size), or 2^32 - 1 for page_size 1
-  int rows_per_wg;   // query rows per workgroup (1 or 4)
+  int rows_per_wg;   // query rows per workgroup (1 or 4; RX_ROWS: the matrix form)
   float* ws;         // splits > 1: [n] max, [n] denominator, [n, d_c] context, n = rows * splits
   int64_t accoff;    // offset of the contexts in ws (floats)
   int log2;          // the maxima are in the exp2 domain

@@ -29,7 +29,6 @@ constexpr int RX_ROWS = 32, RX_KEYS = 32, RX_WAVES = 8, RX_MAX_ND = 3;
 // chain; nine of 64: one SIMD with three waves has too few registers.)
 inline int rx_dim_tiles(int dc) { return (dc + 32 * RX_WAVES - 1) / (32 * RX_WAVES); }
 constexpr float RX_LOG2E = 1.44269504088896340736f;
-constexpr float RX_LARGE = 1e5f;   // scores (exp2 domain) whose rounding reaches 2^-8
 
 __device__ __forceinline__ float rx_max32(float v) {   // over lanes l and l ^ 32 (see xmax16_32)
   float t;

@@ -100,9 +100,10 @@ __device__ __forceinline__ uint32_t e4m3fn_rne(float v) {
 // INT4_RESIDUAL codes of a page of finite values that are not all (nearly) zero: false,
 // and nothing written, for any other page. This kernel is bound by its arithmetic
 // (32,771 pages x 128: 81 us in the plain form with its IEEE divisions, where the other
-// precisions take 36 to 41 us for the same traffic; this form 45 to 51), so here pairs of values stay in packed float16 where the arithmetic is
-// float16 anyway, no value is tested for NaN, and adding 1.5 * 2^10 + 8 (float16) or
-// 1.5 * 2^23 + 8 rounds to the integer, ties to even, and leaves code + 8 in the low byte.
+// precisions take 36 to 42 us for the same traffic; this form 48 to 56, by the box), so
+// here pairs of values stay in packed float16 where the arithmetic is float16 anyway, no
+// value is tested for NaN, and adding 1.5 * 2^10 + 8 (float16) or 1.5 * 2^23 + 8 rounds to
+// the integer, ties to even, and leaves code + 8 in the low byte.
 template <int NL>
 __device__ __forceinline__ bool finite_residual_codes(const h8 (&v)[NL], uint32_t (&out)[NL][2], float& s, float& s2) {
   typedef unsigned short us2 __attribute__((ext_vector_type(2)));
