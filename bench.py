@@ -661,7 +661,7 @@ def run_quantize(args, cpu=None) -> None:
            "config": {"workload": f"{args.config}: {sum(j['src'].shape[0] for j in wl['jobs'])} pages of 16x128 "
                                   f"quantised into 1,048,576-slot K and V pools (6 launches per step)",
                       "algorithmic_bytes": ab},
-           "kernel_source_digest": source_digest(["quantize.hip", "iak_internal.h", "iak_device.h"]),
+           "kernel_source_digest": source_digest(["quantize.hip", "scale_quotient.h", "iak_internal.h", "iak_device.h"]),
            "roofline": {"bound": "hbm", "achieved": round(gbps, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                         "frac": round(gbps / HBM_PEAK_GBPS, 4), "traffic": None}}
     if cpu is not None:
@@ -925,7 +925,7 @@ def run_dense(args) -> None:
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic (seeded N(0,1))",
         "config": {"workload": "dense_attention shapes; value = 8 rows x 8,192 keys x 128 (float16), split over keys"},
-        "kernel_source_digest": source_digest(["dense_attention.hip", "iak_device.h"]),
+        "kernel_source_digest": source_digest(["dense_attention.hip", "dense_matrix.h", "dense_walk.h", "iak_device.h"]),
         "shapes": rows}), flush=True)
 
 
@@ -976,7 +976,7 @@ def run_mla_rows(args) -> None:
         "higher_is_better": False, "scaling": "weak", "vs_baseline": None, "dtype": "f32",
         "data": "synthetic (seeded N(0,1))",
         "config": {"workload": "mla_latent_context shapes; value = 32 sequences x 8,192 latent rows x 576 (float16)"},
-        "kernel_source_digest": source_digest(["mla_rows.hip", "iak_device.h"]),
+        "kernel_source_digest": source_digest(["mla_rows.hip", "mla_rows_matrix.h", "mla_project.h", "iak_device.h"]),
         "shapes": rows}), flush=True)
 
 
@@ -1045,7 +1045,7 @@ def run_fake_quant(args) -> None:
         "data": "synthetic (seeded N(0,1))",
         "config": {"workload": "reconstruction shapes; value = 32 heads x 3 blocks of 1,024 tokens x 256 channels "
                                "(INT8, INT4_RESIDUAL, FP8), split"},
-        "kernel_source_digest": source_digest(["fake_quant.hip"]),
+        "kernel_source_digest": source_digest(["fake_quant.hip", "scale_quotient.h"]),
         "shapes": rows}), flush=True)
 
 

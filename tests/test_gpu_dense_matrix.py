@@ -129,6 +129,27 @@ def test_replays_from_a_graph():
         assert torch.equal(out, want) and not torch.equal(out, eager), i
 
 
+@pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
+def test_short_calls_replay_from_a_graph(dt):
+    """A short call has no workspace of its own, and its second walk runs when a replay's inputs ask
+    for it: finite inputs, an infinity, finite ones again."""
+    from intent_attention import dense_attention
+    q, k, v, g = _qkv(5, (4, 40), 20, 200, 64, 64, dt)
+    qc, kc, vc = q.cuda(), k.cuda(), v.cuda()
+    dense_attention(qc, kc, vc)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = dense_attention(qc, kc, vc)
+    for i in range(4):
+        qc.copy_(torch.randn(q.shape, generator=g).to(DT[dt]))
+        vc[1, 3, 199, 7] = float("inf") if i % 2 else 1.0
+        graph.replay()
+        want = dense_attention(qc, kc, vc)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i
+        assert bool(torch.isposinf(out[1, 3, :, 7]).all()) == bool(i % 2) and int(torch.isinf(out).sum()) == 20 * (i % 2)
+
+
 # rows form (1 row, few pairs), split rows, and the three wave shapes of the matrix form; head
 # dims with and without 16-byte rows
 @pytest.mark.parametrize("dt", ["f16", "bf16", "f32"])
